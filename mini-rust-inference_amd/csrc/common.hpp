@@ -351,6 +351,12 @@ mri_status gemm_ws_get(hipStream_t stream, size_t bytes, void **ptr);
 mri_status launch_q4_0_dequant(const float *x, size_t m, size_t k, const uint8_t *w,
                                size_t n_out, bool ggml_order, float *out, hipStream_t s);
 
+// q4_gemm.hip: the same for more rows (x 16-byte aligned), on the bf16 matrix
+// cores with the f32 activations split exactly.
+bool q4_gemm_supported(size_t m, size_t k, size_t n_out);
+mri_status launch_q4_gemm(const float *x, size_t m, size_t k, const uint8_t *w, size_t n_out,
+                          bool ggml_order, float *out, hipStream_t s);
+
 // capi.cpp: row concatenation of weight handles (whole 16-row tiles, one K)
 // into a new handle, for fused projections that share their input.
 mri_status concat_qmatrix(const mri_qmatrix *const *parts, int n, hipStream_t s,

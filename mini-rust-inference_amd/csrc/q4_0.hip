@@ -1,5 +1,6 @@
-// q4_0.hip — W4A32 Q4_0 GEMV/GEMM on raw GGUF Q4_0 bytes
-// (matmul_q4_0_dequant, ops/matmul/q4_0.rs:94-181).
+// q4_0.hip — W4A32 Q4_0 products of up to 4 rows on raw GGUF Q4_0 bytes
+// (matmul_q4_0_dequant, ops/matmul/q4_0.rs:94-181); more rows go to
+// q4_gemm.hip.
 //
 // The reference dequantizes each block (w = d * (nibble - 8), interleaved
 // nibble order: element 2i = low nibble of byte i, 2i+1 = high nibble,
@@ -278,6 +279,8 @@ mri_status launch_q4(const float *x, size_t m, size_t k, const uint8_t *w, size_
 mri_status launch_q4_0_dequant(const float *x, size_t m, size_t k, const uint8_t *w,
                                size_t n_out, bool ggml_order, float *out, hipStream_t s) {
     if (m == 0 || n_out == 0) return MRI_OK;
+    if (m > 4 && q4_gemm_supported(m, k, n_out))
+        return launch_q4_gemm(x, m, k, w, n_out, ggml_order, out, s);
     return ggml_order ? launch_q4<true>(x, m, k, w, n_out, out, s)
                       : launch_q4<false>(x, m, k, w, n_out, out, s);
 }

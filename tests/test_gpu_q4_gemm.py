@@ -1,0 +1,114 @@
+"""matmul_q4_0_dequant on the matrix cores (more than 4 rows): every tile
+size and K split of its dispatch at the edges of their ranges, in both nibble
+orders, from weights at 2-byte alignment, against the product in 64 bits.
+
+Tolerance: the activations are split exactly and every product is exact, so
+the f32 sums alone round: the entry point's contract (1e-5 of
+max(|result|, sum of |terms|)) per element, and 1e-6 in the 2-norm (about 1e-7
+per rounding of a sum, the roundings of a block's and a row's sums being
+independent)."""
+import numpy as np
+import pytest
+
+import closed_form as CF
+from gpu_util import F32, dev, empty, host, synth_q4_0, torch
+
+pytestmark = pytest.mark.gpu
+
+
+def mri():
+    import mri_qmatmul
+    return mri_qmatmul
+
+
+def at_two_bytes(raw):
+    buf = torch().zeros(raw.size + 2, dtype=torch().uint8, device="cuda")
+    buf[2:] = dev(raw)
+    return buf[2:]
+
+
+def exact(x, raw, n, k):
+    d, q = CF.q4_0_split(raw, n, k)
+    w = np.repeat(d.astype(np.float64), 32, axis=1) * q
+    return x.astype(np.float64) @ w.T
+
+
+def check(got, x, raw, n, k):
+    ref = exact(x, raw, n, k)
+    err = np.abs(got.astype(np.float64) - ref)
+    scale = np.maximum(np.abs(ref), CF.q4_0_terms_abs_sum(x, raw, n, k))
+    assert np.all(err <= 1e-5 * scale), float(np.max(err / scale))
+    assert np.linalg.norm(err) <= 1e-6 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (5, 1, 32), (16, 17, 288), (7, 6200, 544),          # 16-row tiles, narrow and wide
+    (17, 33, 32), (32, 31, 288), (18, 8300, 320),       # 32-row tiles
+    (33, 129, 96), (64, 127, 1056), (65, 300, 2048),    # 64 x 128 and its K split
+    (130, 1000, 4096), (200, 515, 11008),               # 128-row tiles in K parts
+    (513, 4100, 256), (1100, 777, 64)])
+@pytest.mark.parametrize("ggml", [False, True])
+def test_rows_and_tile_edges(m, n, k, ggml):
+    rng = np.random.default_rng(m * 7 + n + k)
+    raw = synth_q4_0(rng, n, k)
+    x = (rng.standard_normal((m, k)) * np.exp(rng.standard_normal(k))).astype(F32)
+    out = torch().full((m + 1, n), 7.0, device="cuda")
+    disk = CF.q4_0_interleaved_to_ggml(raw) if ggml else raw
+    order = mri().Q4_ORDER_GGML if ggml else mri().Q4_ORDER_INTERLEAVED
+    for w in (dev(disk), at_two_bytes(disk)):
+        mri().matmul_q4_0_dequant_ordered(dev(x), w, n, k, order, out[:m])
+        got = host(out)
+        check(got[:m], x, raw, n, k)
+        assert np.all(got[m] == 7.0)
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e30])
+def test_wide_range_of_activations(scale):
+    """Rows whose values span 2^24 at both ends of the f32 range: the three
+    planes carry all of them (for the small ones, down to the last plane's
+    2^-133, far below the bound)."""
+    rng = np.random.default_rng(5)
+    m, n, k = 40, 64, 512
+    raw = synth_q4_0(rng, n, k)
+    x = (rng.standard_normal((m, k)) * np.exp2(rng.integers(-12, 13, (m, k))) * scale).astype(F32)
+    out = empty((m, n), torch().float32)
+    mri().matmul_q4_0_dequant(dev(x), dev(raw), n, k, out)
+    check(host(out), x, raw, n, k)
+
+
+def test_nonfinite_activations_stay_in_their_rows():
+    rng = np.random.default_rng(6)
+    m, n, k = 9, 40, 96
+    raw = synth_q4_0(rng, n, k)
+    x = rng.standard_normal((m, k)).astype(F32)
+    x[2, 5], x[4, 40], x[7, 95] = np.inf, -np.inf, np.nan
+    out = empty((m, n), torch().float32)
+    mri().matmul_q4_0_dequant(dev(x), dev(raw), n, k, out)
+    got = host(out)
+    bad = np.array([2, 4, 7])
+    assert not np.isfinite(got[bad]).any()
+    good = np.setdiff1d(np.arange(m), bad)
+    check(got[good], x[good], raw, n, k)
+
+
+def test_captured_call_needs_no_workspace():
+    """A shape that splits K in an eager call is captured on a stream the
+    library has not seen, and its replays match."""
+    t = torch()
+    rng = np.random.default_rng(8)
+    m, n, k = 128, 512, 4096
+    raw = synth_q4_0(rng, n, k)
+    x = rng.standard_normal((m, k)).astype(F32)
+    xd, w, out = dev(x), dev(raw), empty((m, n), t.float32)
+    mri().matmul_q4_0_dequant(xd, w, n, k, out)
+    check(host(out), x, raw, n, k)
+    t.cuda.synchronize()
+    s = t.cuda.Stream()
+    g = t.cuda.CUDAGraph()
+    with t.cuda.graph(g, stream=s):
+        mri().matmul_q4_0_dequant(xd, w, n, k, out)
+    for _ in range(3):
+        out.fill_(0)
+        g.replay()
+        check(host(out), x, raw, n, k)
+        xd.copy_(xd * 1.0)
