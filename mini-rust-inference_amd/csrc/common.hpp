@@ -351,9 +351,7 @@ mri_status gemm_ws_get(hipStream_t stream, size_t bytes, void **ptr);
 mri_status launch_q4_0_dequant(const float *x, size_t m, size_t k, const uint8_t *w,
                                size_t n_out, bool ggml_order, float *out, hipStream_t s);
 
-// q4_gemm.hip: the same for more rows (x 16-byte aligned), on the bf16 matrix
-// cores with the f32 activations split exactly.
-bool q4_gemm_supported(size_t m, size_t k, size_t n_out);
+// q4_gemm.hip: the same (k > 0, x 16-byte aligned) for any rows, tiled.
 mri_status launch_q4_gemm(const float *x, size_t m, size_t k, const uint8_t *w, size_t n_out,
                           bool ggml_order, float *out, hipStream_t s);
 

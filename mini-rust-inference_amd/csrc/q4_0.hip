@@ -4,133 +4,198 @@
 //
 // The reference dequantizes each block (w = d * (nibble - 8), interleaved
 // nibble order: element 2i = low nibble of byte i, 2i+1 = high nibble,
-// q4_0.rs:59-68) and accumulates x*w in f32 over K.  Here the dequantization
-// happens in registers and the sum is regrouped per block:
-//   sum_b d_b * (sum_e x_e * nib_e - 8 * sum_e x_e)
-// which differs from the sequential sum only by rounding (the documented
-// 1e-5 * max(|ref|, sum|terms|) contract).
+// q4_0.rs:59-68) and accumulates x*w in f32 over K.  Here the sum is
+// regrouped per block, which differs from the sequential sum only by rounding
+// (the documented 1e-5 * max(|ref|, sum|terms|) contract).
 //
 // Two forms.
 //
+// k_q4_0_gemv (1-4 rows, any 2-byte aligned layout): the matrix cores, with
+// the f32 activations split exactly into three bf16 planes (q4_common.hpp).
+// A workgroup takes 16 channels and its waves split K in laps of 4 blocks:
+// lane (r, g) loads block 4 lap + g of channel r, 18 contiguous bytes, and
+// holds the block's 32 quants as the B operands of four MFMAs.  All 64 lanes
+// hold different k then, so row 4g + p of the A operand carries plane p of
+// the activations of block 4 lap + g and is zero elsewhere; the four MFMAs
+// add up to register p of lane (r, g) = plane p's sum of its own block, which
+// it adds (smallest first) and scales by the d that it loaded.  The planes
+// are split once per workgroup into LDS.  Bound: the unpacking (2.6 VALU
+// operations a weight) and its loads, 72-byte pieces of 16 rows.  It took
+// 1 x 4128 x 11008 from 23.4 to 10.4 us (the earlier two-lanes-a-block f32
+// kernel), 2 x 4128 x 8000 from 33.1 to 9.2 and 4 x 992 x 512 from 12.9 to
+// 4.4; against the staged form below 2 x 4096 x 11008 16.8 -> 13.6.  More
+// laps in flight, or a wave's laps adjacent, were slower (1 x 4096 x 11008:
+// 14-20 us), as was staging the rows through LDS by DMA (12.7-19).
+//
 // k_q4_0_lds (16-byte aligned weights, K % 256 == 0, so that every row
-// starts on 16 bytes; M <= 4): a workgroup takes R consecutive weight rows,
+// starts on 16 bytes; one row): a workgroup takes R consecutive weight rows,
 // one contiguous byte range, and moves them to LDS with 16-byte loads (all
 // in flight at once); the activations are read from L2.  Lane l of a step
 // covers elements 8*(l%4) .. +8 of block l/4 (4 quant
 // bytes: low nibble = even element): it reads its 8 activations once and
 // applies them to each of the wave's R/4 rows as d * (sum x*nib - 8 * sum x)
-// (the regrouping below; the activation sum is shared by the rows).  Lane
-// partials are added by a wave reduction.
-//
-// k_q4_0_dequant (any 2-byte aligned layout): one wave per weight row, two
-// lanes per block (16 elements each), with the sum regrouped per block as
-// sum_b d_b * (sum_e x_e * nib_e - 8 * sum_e x_e).
+// (the activation sum is shared by the rows).  Lane partials are added by a
+// wave reduction.
 //
 // GG (an option without a reference counterpart): upstream GGML's nibble
 // order, element i = low nibble of byte i and element i + 16 = its high
-// nibble (llama.cpp Q4_0 files); the lanes then read the bytes of their
-// elements and take one nibble of each.
+// nibble (llama.cpp Q4_0 files).
 #include <algorithm>
 
 #include "common.hpp"
+#include "q4_common.hpp"
 
 namespace mri {
 namespace {
 
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef unsigned u4 __attribute__((ext_vector_type(4)));
+struct __attribute__((packed, aligned(4))) Words4 {
+    unsigned v[4];
+};
+
 constexpr int kThreads = 256;
-constexpr int kRowsPerWave = 4;
+constexpr int kMaxLds = 160 * 1024;
 
-
-// 8 quant bytes (two u32 words) against 16 activations: returns
-// sum_e x_e * nib_e for the interleaved order.
-__device__ inline float nib_dot(unsigned w0, unsigned w1, const float *x) {
-    float s = 0.0f;
-    const unsigned lo0 = w0 & 0x0F0F0F0Fu, hi0 = (w0 >> 4) & 0x0F0F0F0Fu;
-    const unsigned lo1 = w1 & 0x0F0F0F0Fu, hi1 = (w1 >> 4) & 0x0F0F0F0Fu;
-    s = fmaf(x[0], (float)(lo0 & 0xFF), s);
-    s = fmaf(x[1], (float)(hi0 & 0xFF), s);
-    s = fmaf(x[2], (float)((lo0 >> 8) & 0xFF), s);
-    s = fmaf(x[3], (float)((hi0 >> 8) & 0xFF), s);
-    s = fmaf(x[4], (float)((lo0 >> 16) & 0xFF), s);
-    s = fmaf(x[5], (float)((hi0 >> 16) & 0xFF), s);
-    s = fmaf(x[6], (float)(lo0 >> 24), s);
-    s = fmaf(x[7], (float)(hi0 >> 24), s);
-    s = fmaf(x[8], (float)(lo1 & 0xFF), s);
-    s = fmaf(x[9], (float)(hi1 & 0xFF), s);
-    s = fmaf(x[10], (float)((lo1 >> 8) & 0xFF), s);
-    s = fmaf(x[11], (float)((hi1 >> 8) & 0xFF), s);
-    s = fmaf(x[12], (float)((lo1 >> 16) & 0xFF), s);
-    s = fmaf(x[13], (float)((hi1 >> 16) & 0xFF), s);
-    s = fmaf(x[14], (float)(lo1 >> 24), s);
-    s = fmaf(x[15], (float)(hi1 >> 24), s);
-    return s;
+// LDS of k_q4_0_gemv: [M][3 planes][4 Q blocks][64 bytes] and a 16-byte zero
+// line; the reduction's M * NW * 16 floats fit in it (NW <= 16, Q >= 1: 768 M
+// bytes and more).
+size_t q4_gemv_lds(int m, int nw, size_t k) {
+    const size_t q = (k / 32 + 3) / 4;
+    return std::max((size_t)m * 3 * q * 256 + 16, (size_t)m * nw * 64);
 }
 
-// 16 bytes (four u32 words) against 16 activations, GGML order: element e
-// is nibble `shift` / 4 of byte e.
-__device__ inline float nib_dot_ggml(const unsigned (&wd)[4], int shift, const float *x) {
-    float s = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e)
-        s = fmaf(x[e], (float)((wd[e >> 2] >> (8 * (e & 3) + shift)) & 0xFu), s);
-    return s;
-}
+template <int M, int NW, bool GG>
+__global__ __launch_bounds__(NW * 64) void k_q4_0_gemv(const float *__restrict__ x, int K,
+                                                       const uint8_t *__restrict__ w, int N,
+                                                       float *__restrict__ out) {
+    constexpr int NT = NW * 64;
+    extern __shared__ u4 s_x[];
+    const int t = threadIdx.x, l = t & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nb = K / 32, Q = (nb + 3) / 4;
+    const int r = l & 15, g = l >> 4;
+    const int plane = Q * 16;  // 16-byte pieces
+    const int zero = M * 3 * plane;
+    // channels past N read the last one (not stored)
+    const uint8_t *row = w + (size_t)min(16 * (int)blockIdx.x + r, N - 1) * nb * kQ4Bytes;
 
-template <bool GG>
-__global__ __launch_bounds__(kThreads) void k_q4_0_dequant(
-    const float *__restrict__ x, int M, int K, const uint16_t *__restrict__ w,
-    int N, float *__restrict__ out) {
-    const int lane = threadIdx.x & 63;
-    const int wave = (blockIdx.x * kThreads + threadIdx.x) >> 6;
-    const int n_waves = (gridDim.x * kThreads) >> 6;
-    const int nb = K / 32;
-    const int half = lane & 1;
-    const size_t row_u16 = (size_t)nb * (kQ4Bytes / 2);
-    for (int n = wave; n < N; n += n_waves) {
-        const uint16_t *row = w + (size_t)n * row_u16;
-        for (int m = 0; m < M; ++m) {
-            const float *xr = x + (size_t)m * K;
-            float acc = 0.0f;
-            for (int b = lane >> 1; b < nb; b += 32) {
-                const uint16_t *blk = row + (size_t)b * (kQ4Bytes / 2);
-                const float d = f16_bits_to_f32(blk[0]);
-                const float4 *xv = reinterpret_cast<const float4 *>(xr + b * 32 + half * 16);
-                float xe[16];
+    // The 18 bytes of this lane's block of a lap (blocks past the end: the
+    // last one, counted as zero): the 4-byte aligned words around its quants
+    // and, as 2-byte loads that stay inside the block, the last quants and
+    // the scale.
+    unsigned q[5], d;
+    auto load = [&](int lap) __attribute__((always_inline)) {
+        const uint8_t *p = row + (size_t)min(4 * lap + g, nb - 1) * kQ4Bytes;
+        const Words4 v = *reinterpret_cast<const Words4 *>(((uintptr_t)p + 2) & ~(uintptr_t)3);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float4 v = xv[j];
-                    xe[4 * j] = v.x;
-                    xe[4 * j + 1] = v.y;
-                    xe[4 * j + 2] = v.z;
-                    xe[4 * j + 3] = v.w;
-                }
-                float xs = 0.0f;
+        for (int i = 0; i < 4; ++i) q[i] = v.v[i];
+        q[4] = *reinterpret_cast<const uint16_t *>(p + 16);
+        d = *reinterpret_cast<const uint16_t *>(p);
+    };
+    // Unit u of a row: the 8 activations of word j = u % 4 (4 quant bytes) of
+    // block u / 4; LDS holds them in the word's nibble order, low nibbles
+    // first.
+    auto get = [&](int m, int u, f4 &a, f4 &b) __attribute__((always_inline)) {
+        const int blk = min(u >> 2, nb - 1), j = u & 3;
+        const float *p = x + (size_t)m * K + 32 * blk;
+        a = *reinterpret_cast<const f4 *>(p + (GG ? 4 * j : 8 * j));
+        b = *reinterpret_cast<const f4 *>(p + (GG ? 16 + 4 * j : 8 * j + 4));
+    };
+    auto put = [&](int m, int u, f4 a, f4 b) __attribute__((always_inline)) {
+        if (u >= 4 * nb) a = b = f4{0, 0, 0, 0};
+        f4 lo = GG ? a : f4{a[0], a[2], b[0], b[2]};
+        f4 hi = GG ? b : f4{a[1], a[3], b[1], b[3]};
 #pragma unroll
-                for (int j = 0; j < 16; ++j) xs += xe[j];
-                float s;
-                if constexpr (GG) {
-                    // elements 16 half .. +15: nibble `half` of all 16 bytes
-                    unsigned wd[4];
+        for (int p = 0; p < 3; ++p) {
+            s_x[(m * 3 + p) * plane + u] = u4{q4_top16(lo[0], lo[1]), q4_top16(lo[2], lo[3]),
+                                              q4_top16(hi[0], hi[1]), q4_top16(hi[2], hi[3])};
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        wd[i] = (unsigned)blk[1 + 2 * i] | ((unsigned)blk[2 + 2 * i] << 16);
-                    s = nib_dot_ggml(wd, 4 * half, xe);
-                } else {
-                    const uint16_t *qs = blk + 1 + half * 4;
-                    const unsigned w0 = (unsigned)qs[0] | ((unsigned)qs[1] << 16);
-                    const unsigned w1 = (unsigned)qs[2] | ((unsigned)qs[3] << 16);
-                    s = nib_dot(w0, w1, xe);
-                }
-                acc = fmaf(d, fmaf(-8.0f, xs, s), acc);
+            for (int e = 0; e < 4; ++e) {
+                lo[e] -= q4_cut(lo[e]);
+                hi[e] -= q4_cut(hi[e]);
             }
-            for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-            if (lane == 0) out[(size_t)m * N + n] = acc;
         }
+    };
+    const int units = 16 * Q;
+    f4 xa[M], xb[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m) get(m, min(t, units - 1), xa[m], xb[m]);
+    load(wv);
+    if (t == 0) s_x[zero] = u4{0, 0, 0, 0};
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+        if (t < units) put(m, t, xa[m], xb[m]);
+    for (int u = t + NT; u < units; u += NT) {
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            f4 a, b;
+            get(m, u, a, b);
+            put(m, u, a, b);
+        }
+    }
+    // LDS only: the weight loads stay in flight
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+
+    float acc[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m) acc[m] = 0.0f;
+    const bool on = (r >> 2) == g && (r & 3) < 3;
+    const int st = on ? 1 : 0;
+    for (int lap = wv; lap < Q; lap += NW) {
+        const int blk = 4 * lap + g;
+        const float ds = blk < nb ? f16_bits_to_f32(d) : 0.0f;
+        // quants at 2 bytes past a word: shifted into place
+        const uintptr_t p = (uintptr_t)row + (uintptr_t)(min(blk, nb - 1) * (size_t)kQ4Bytes);
+        const unsigned sh = 2u - ((unsigned)p & 2u);
+        bf8 b[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float lo[4], hi[4];
+            q4_quants(__builtin_amdgcn_alignbyte(q[j + 1], q[j], sh), lo, hi);
+            b[j] = __builtin_bit_cast(
+                bf8, u4{q4_top16(lo[0], lo[1]), q4_top16(lo[2], lo[3]), q4_top16(hi[0], hi[1]),
+                        q4_top16(hi[2], hi[3])});
+        }
+        load(lap + NW);
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            f4 c{0, 0, 0, 0};
+            const int ai = on ? (m * 3 + (r & 3)) * plane + 4 * g + 16 * lap : zero;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    __builtin_bit_cast(bf8, s_x[ai + st * j]), b[j], c, 0, 0, 0);
+            acc[m] = __builtin_fmaf((c[2] + c[1]) + c[0], ds, acc[m]);
+        }
+    }
+    // the four lane groups' blocks, then the waves' laps in wave order
+    __syncthreads();
+    float *red = reinterpret_cast<float *>(s_x);
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+        acc[m] += __shfl_xor(acc[m], 16);
+        acc[m] += __shfl_xor(acc[m], 32);
+        if (l < 16) red[(m * NW + wv) * 16 + l] = acc[m];
+    }
+    __syncthreads();
+    if (t < 16 * M) {
+        const int m = t >> 4, n = 16 * blockIdx.x + (t & 15);
+        float s = red[m * NW * 16 + (t & 15)];
+#pragma unroll
+        for (int v = 1; v < NW; ++v) s += red[(m * NW + v) * 16 + (t & 15)];
+        if (n < N) out[(size_t)m * N + n] = s;
     }
 }
 
+__global__ __launch_bounds__(kThreads) void k_q4_0_empty(size_t n, float *__restrict__ out) {
+    const size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x;
+    if (i < n) out[i] = 0.0f;
+}
+
 template <int R, bool GG>
-__global__ __launch_bounds__(kThreads) void k_q4_0_lds(const float *__restrict__ x, int M, int K,
+__global__ __launch_bounds__(kThreads) void k_q4_0_lds(const float *__restrict__ x, int K,
                                                        const uint8_t *__restrict__ w, int N,
                                                        float *__restrict__ out) {
     constexpr int RW = R / 4;  // rows per wave
@@ -158,120 +223,152 @@ __global__ __launch_bounds__(kThreads) void k_q4_0_lds(const float *__restrict__
     __syncthreads();
     const int steps = (nb * 4 + 63) / 64;
     // rows past `rows` read stale LDS and are never stored
-    for (int m = 0; m < M; ++m) {
-        const float *xm = x + (size_t)m * K;
-        float acc[RW];
+    float acc[RW];
 #pragma unroll
-        for (int r = 0; r < RW; ++r) acc[r] = 0.0f;
-        for (int st = 0; st < steps; ++st) {
-            const int idx = st * 64 + lane, p = idx & 3;
-            const bool ok = (idx >> 2) < nb;
-            const int b = ok ? idx >> 2 : nb - 1;
-            const float4 *xv = reinterpret_cast<const float4 *>(xm + 32 * b + 8 * p);
-            float4 xa = xv[0], xb = xv[1];
-            if (!ok) xa = xb = float4{0, 0, 0, 0};
-            float dq[RW];
-            unsigned lo[RW], hi[RW];
-#pragma unroll
-            for (int r = 0; r < RW; ++r) {
-                const uint8_t *blk = s_w + (size_t)(wv * RW + r) * row_bytes + b * kQ4Bytes;
-                dq[r] = f16_bits_to_f32(*reinterpret_cast<const uint16_t *>(blk));
-                if constexpr (GG) {
-                    // elements 8p .. 8p+7: nibble p / 2 of bytes 8 (p % 2) .. +7,
-                    // regrouped into the (even, odd) element words below
-                    const uint16_t *qs = reinterpret_cast<const uint16_t *>(blk + 2 + 8 * (p & 1));
-                    const int sh = 4 * (p >> 1);
-                    const unsigned a0 = ((unsigned)qs[0] | ((unsigned)qs[1] << 16)) >> sh;
-                    const unsigned a1 = ((unsigned)qs[2] | ((unsigned)qs[3] << 16)) >> sh;
-                    // a0 bytes = elements 0..3, a1 bytes = elements 4..7
-                    const unsigned e0 = a0 & 0x0F0F0F0Fu, e1 = a1 & 0x0F0F0F0Fu;
-                    lo[r] = (e0 & 0xFFu) | ((e0 >> 8) & 0xFF00u) | ((e1 << 16) & 0xFF0000u) |
-                            ((e1 << 8) & 0xFF000000u);          // elements 0, 2, 4, 6
-                    hi[r] = ((e0 >> 8) & 0xFFu) | ((e0 >> 16) & 0xFF00u) |
-                            ((e1 << 8) & 0xFF0000u) | (e1 & 0xFF000000u);  // 1, 3, 5, 7
-                } else {
-                    const unsigned q =
-                        (unsigned)*reinterpret_cast<const uint16_t *>(blk + 2 + 4 * p) |
-                        ((unsigned)*reinterpret_cast<const uint16_t *>(blk + 4 + 4 * p) << 16);
-                    lo[r] = q & 0x0F0F0F0Fu;          // elements 0, 2, 4, 6 (low nibbles)
-                    hi[r] = (q >> 4) & 0x0F0F0F0Fu;   // elements 1, 3, 5, 7
-                }
-            }
-            // d * sum_e x_e * (nib_e - 8) = d * (sum_e x_e * nib_e - 8 * sum_e x_e);
-            // the activation sum is shared by the wave's rows, and the rows'
-            // chains are interleaved
-            const float xs = ((xa.x + xa.y) + (xa.z + xa.w)) + ((xb.x + xb.y) + (xb.z + xb.w));
-            float sn[RW];
-#pragma unroll
-            for (int r = 0; r < RW; ++r) sn[r] = xa.x * (float)(lo[r] & 0xFF);
-#pragma unroll
-            for (int r = 0; r < RW; ++r) sn[r] = fmaf(xa.y, (float)(hi[r] & 0xFF), sn[r]);
-#pragma unroll
-            for (int r = 0; r < RW; ++r) sn[r] = fmaf(xa.z, (float)((lo[r] >> 8) & 0xFF), sn[r]);
-#pragma unroll
-            for (int r = 0; r < RW; ++r) sn[r] = fmaf(xa.w, (float)((hi[r] >> 8) & 0xFF), sn[r]);
-#pragma unroll
-            for (int r = 0; r < RW; ++r) sn[r] = fmaf(xb.x, (float)((lo[r] >> 16) & 0xFF), sn[r]);
-#pragma unroll
-            for (int r = 0; r < RW; ++r) sn[r] = fmaf(xb.y, (float)((hi[r] >> 16) & 0xFF), sn[r]);
-#pragma unroll
-            for (int r = 0; r < RW; ++r) sn[r] = fmaf(xb.z, (float)(lo[r] >> 24), sn[r]);
-#pragma unroll
-            for (int r = 0; r < RW; ++r) sn[r] = fmaf(xb.w, (float)(hi[r] >> 24), sn[r]);
-#pragma unroll
-            for (int r = 0; r < RW; ++r) acc[r] = fmaf(dq[r], fmaf(-8.0f, xs, sn[r]), acc[r]);
-        }
+    for (int r = 0; r < RW; ++r) acc[r] = 0.0f;
+    for (int st = 0; st < steps; ++st) {
+        const int idx = st * 64 + lane, p = idx & 3;
+        const bool ok = (idx >> 2) < nb;
+        const int b = ok ? idx >> 2 : nb - 1;
+        const float4 *xv = reinterpret_cast<const float4 *>(x + 32 * b + 8 * p);
+        float4 xa = xv[0], xb = xv[1];
+        if (!ok) xa = xb = float4{0, 0, 0, 0};
+        float dq[RW];
+        unsigned lo[RW], hi[RW];
 #pragma unroll
         for (int r = 0; r < RW; ++r) {
-            float v = acc[r];
-            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-            const int row = wv * RW + r;
-            if (lane == 0 && row < rows) out[(size_t)m * N + n0 + row] = v;
+            const uint8_t *blk = s_w + (size_t)(wv * RW + r) * row_bytes + b * kQ4Bytes;
+            dq[r] = f16_bits_to_f32(*reinterpret_cast<const uint16_t *>(blk));
+            if constexpr (GG) {
+                // elements 8p .. 8p+7: nibble p / 2 of bytes 8 (p % 2) .. +7,
+                // regrouped into the (even, odd) element words below
+                const uint16_t *qs = reinterpret_cast<const uint16_t *>(blk + 2 + 8 * (p & 1));
+                const int sh = 4 * (p >> 1);
+                const unsigned a0 = ((unsigned)qs[0] | ((unsigned)qs[1] << 16)) >> sh;
+                const unsigned a1 = ((unsigned)qs[2] | ((unsigned)qs[3] << 16)) >> sh;
+                // a0 bytes = elements 0..3, a1 bytes = elements 4..7
+                const unsigned e0 = a0 & 0x0F0F0F0Fu, e1 = a1 & 0x0F0F0F0Fu;
+                lo[r] = (e0 & 0xFFu) | ((e0 >> 8) & 0xFF00u) | ((e1 << 16) & 0xFF0000u) |
+                        ((e1 << 8) & 0xFF000000u);          // elements 0, 2, 4, 6
+                hi[r] = ((e0 >> 8) & 0xFFu) | ((e0 >> 16) & 0xFF00u) |
+                        ((e1 << 8) & 0xFF0000u) | (e1 & 0xFF000000u);  // 1, 3, 5, 7
+            } else {
+                const unsigned q =
+                    (unsigned)*reinterpret_cast<const uint16_t *>(blk + 2 + 4 * p) |
+                    ((unsigned)*reinterpret_cast<const uint16_t *>(blk + 4 + 4 * p) << 16);
+                lo[r] = q & 0x0F0F0F0Fu;          // elements 0, 2, 4, 6 (low nibbles)
+                hi[r] = (q >> 4) & 0x0F0F0F0Fu;   // elements 1, 3, 5, 7
+            }
         }
+        // d * sum_e x_e * (nib_e - 8) = d * (sum_e x_e * nib_e - 8 * sum_e x_e);
+        // the activation sum is shared by the wave's rows, and the rows'
+        // chains are interleaved
+        const float xs = ((xa.x + xa.y) + (xa.z + xa.w)) + ((xb.x + xb.y) + (xb.z + xb.w));
+        float sn[RW];
+#pragma unroll
+        for (int r = 0; r < RW; ++r) sn[r] = xa.x * (float)(lo[r] & 0xFF);
+#pragma unroll
+        for (int r = 0; r < RW; ++r) sn[r] = fmaf(xa.y, (float)(hi[r] & 0xFF), sn[r]);
+#pragma unroll
+        for (int r = 0; r < RW; ++r) sn[r] = fmaf(xa.z, (float)((lo[r] >> 8) & 0xFF), sn[r]);
+#pragma unroll
+        for (int r = 0; r < RW; ++r) sn[r] = fmaf(xa.w, (float)((hi[r] >> 8) & 0xFF), sn[r]);
+#pragma unroll
+        for (int r = 0; r < RW; ++r) sn[r] = fmaf(xb.x, (float)((lo[r] >> 16) & 0xFF), sn[r]);
+#pragma unroll
+        for (int r = 0; r < RW; ++r) sn[r] = fmaf(xb.y, (float)((hi[r] >> 16) & 0xFF), sn[r]);
+#pragma unroll
+        for (int r = 0; r < RW; ++r) sn[r] = fmaf(xb.z, (float)(lo[r] >> 24), sn[r]);
+#pragma unroll
+        for (int r = 0; r < RW; ++r) sn[r] = fmaf(xb.w, (float)(hi[r] >> 24), sn[r]);
+#pragma unroll
+        for (int r = 0; r < RW; ++r) acc[r] = fmaf(dq[r], fmaf(-8.0f, xs, sn[r]), acc[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+        float v = acc[r];
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+        const int row = wv * RW + r;
+        if (lane == 0 && row < rows) out[n0 + row] = v;
     }
 }
 
 size_t q4_lds_bytes(int r, size_t k) { return (size_t)r * (k / 32) * kQ4Bytes; }
 
 template <int R, bool GG>
-mri_status launch_lds(const float *x, size_t m, size_t k, const uint8_t *w, size_t n_out,
+mri_status launch_lds(const float *x, size_t k, const uint8_t *w, size_t n_out,
                       float *out, hipStream_t s) {
     static DeviceOnce attr;
     MRI_HIP(attr.run([](int) {
         return hipFuncSetAttribute(reinterpret_cast<const void *>(&k_q4_0_lds<R, GG>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
     }));
     hipLaunchKernelGGL((k_q4_0_lds<R, GG>), dim3((unsigned)((n_out + R - 1) / R)),
-                       dim3(kThreads), q4_lds_bytes(R, k), s, x, (int)m, (int)k, w, (int)n_out,
-                       out);
+                       dim3(kThreads), q4_lds_bytes(R, k), s, x, (int)k, w, (int)n_out, out);
     MRI_LAUNCHED("k_q4_0_lds");
     return MRI_OK;
+}
+
+template <int M, int NW, bool GG>
+mri_status launch_gemv(const float *x, size_t k, const uint8_t *w, size_t n_out, float *out,
+                       hipStream_t s) {
+    static DeviceOnce attr;
+    MRI_HIP(attr.run([](int) {
+        return hipFuncSetAttribute(reinterpret_cast<const void *>(&k_q4_0_gemv<M, NW, GG>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
+    }));
+    hipLaunchKernelGGL((k_q4_0_gemv<M, NW, GG>), dim3((unsigned)((n_out + 15) / 16)),
+                       dim3(NW * 64), q4_gemv_lds(M, NW, k), s, x, (int)k, w, (int)n_out, out);
+    MRI_LAUNCHED("k_q4_0_gemv");
+    return MRI_OK;
+}
+
+template <int NW, bool GG>
+mri_status launch_gemv_rows(const float *x, size_t m, size_t k, const uint8_t *w, size_t n_out,
+                            float *out, hipStream_t s) {
+    switch (m) {
+    case 1: return launch_gemv<1, NW, GG>(x, k, w, n_out, out, s);
+    case 2: return launch_gemv<2, NW, GG>(x, k, w, n_out, out, s);
+    case 3: return launch_gemv<3, NW, GG>(x, k, w, n_out, out, s);
+    default: return launch_gemv<4, NW, GG>(x, k, w, n_out, out, s);
+    }
 }
 
 template <bool GG>
 mri_status launch_q4(const float *x, size_t m, size_t k, const uint8_t *w, size_t n_out,
                      float *out, hipStream_t s) {
-    // the staged form: 16-byte aligned rows (K % 256 == 0) and operands, and
-    // at most 64 KiB of LDS per workgroup (several workgroups per CU)
+    if (k == 0) {
+        const size_t n = m * n_out;
+        hipLaunchKernelGGL(k_q4_0_empty, dim3((unsigned)((n + kThreads - 1) / kThreads)),
+                           dim3(kThreads), 0, s, n, out);
+        MRI_LAUNCHED("k_q4_0_empty");
+        return MRI_OK;
+    }
+    const size_t cus = (size_t)std::max(device_cus(), 1), tiles = (n_out + 15) / 16;
+    const bool few = 2 * tiles <= 3 * cus;  // 16-channel workgroups fit about one a CU
+    // the staged form: 16-byte aligned rows (K % 256 == 0) and operands
     const bool al = ((uintptr_t)w & 15) == 0 && ((uintptr_t)x & 15) == 0 && k % 256 == 0;
-    if (al && m <= 4 && k <= (1u << 16) && n_out <= (1u << 30)) {
+    if (al && m == 1 && n_out <= (1u << 30) && !(few && k >= 8192)) {
         // rows per workgroup: 8, or 4 where 8 rows exceed ~40 KiB of LDS.
         // Measured at K = 4096 (us per call): 8 rows 11.8 (N = 11008) and
         // 6.4 (N = 4096), against 13.1 and 8.4 for 16 rows and 12.7 and 6.4
         // for 4 (more workgroups per CU overlap one's loads with another's
-        // arithmetic)
-        if (q4_lds_bytes(8, k) <= 40 * 1024) return launch_lds<8, GG>(x, m, k, w, n_out, out, s);
-        if (q4_lds_bytes(4, k) <= 48 * 1024) return launch_lds<4, GG>(x, m, k, w, n_out, out, s);
+        // arithmetic).  k_q4_0_gemv takes 13.3 and 7.0 there, its 16
+        // channels' loads being 72-byte pieces; on few channels and a long K
+        // it is the faster one (11008 -> 4096: 10.1 against 12.9, 16 waves).
+        if (q4_lds_bytes(8, k) <= 40 * 1024) return launch_lds<8, GG>(x, k, w, n_out, out, s);
+        if (q4_lds_bytes(4, k) <= 48 * 1024) return launch_lds<4, GG>(x, k, w, n_out, out, s);
     }
-    const size_t waves = (n_out + kRowsPerWave - 1) / kRowsPerWave;
-    size_t grid = (waves + (kThreads / 64) - 1) / (kThreads / 64);
-    if (grid < 1) grid = 1;
-    if (grid > 65535) grid = 65535;
-    hipLaunchKernelGGL((k_q4_0_dequant<GG>), dim3((unsigned)grid), dim3(kThreads), 0, s,
-                       x, (int)m, (int)k, reinterpret_cast<const uint16_t *>(w),
-                       (int)n_out, out);
-    MRI_LAUNCHED("k_q4_0_dequant");
-    return MRI_OK;
+    // Rows 3 and 4 on many channels go to the tiled kernel, which unpacks
+    // each weight once for 16 rows and streams (4 x 4096 x 11008 20.0 us
+    // against 23.6; at N = 4096 10.6 against 8.9), as do rows that LDS does
+    // not hold.
+    const int nw = k >= 8192 && few ? 16 : 8;
+    if (n_out <= (1u << 30) && k <= (1u << 20) && (m <= 2 || (m <= 4 && few)) &&
+        q4_gemv_lds((int)m, nw, k) <= (size_t)kMaxLds)
+        return nw == 16 ? launch_gemv_rows<16, GG>(x, m, k, w, n_out, out, s)
+                        : launch_gemv_rows<8, GG>(x, m, k, w, n_out, out, s);
+    return launch_q4_gemm(x, m, k, w, n_out, GG, out, s);
 }
 
 }  // namespace
@@ -279,8 +376,6 @@ mri_status launch_q4(const float *x, size_t m, size_t k, const uint8_t *w, size_
 mri_status launch_q4_0_dequant(const float *x, size_t m, size_t k, const uint8_t *w,
                                size_t n_out, bool ggml_order, float *out, hipStream_t s) {
     if (m == 0 || n_out == 0) return MRI_OK;
-    if (m > 4 && q4_gemm_supported(m, k, n_out))
-        return launch_q4_gemm(x, m, k, w, n_out, ggml_order, out, s);
     return ggml_order ? launch_q4<true>(x, m, k, w, n_out, out, s)
                       : launch_q4<false>(x, m, k, w, n_out, out, s);
 }

@@ -4,9 +4,8 @@
 //
 //   out[m, n] = sum_b d[n, b] * sum_{k in block b} x[m, k] * (nib[n, k] - 8)
 //
-// An f32 value is exactly the sum of three bf16 values: its leading 8
-// significand bits, the next 8 and the last 8, each cut off (not rounded)
-// from what the ones before leave.  A quant (-8 .. 7) is a bf16 value too,
+// An f32 value is exactly the sum of three bf16 values (q4_common.hpp).  A
+// quant (-8 .. 7) is a bf16 value too,
 // so every product of the three planes with the quants is exact, and
 // v_mfma_f32_16x16x32_bf16 adds them in f32: three MFMAs a block (smallest
 // plane first), then one FMA with the block's scale.  Infinities and NaNs
@@ -32,6 +31,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "q4_common.hpp"
 
 namespace mri {
 namespace {
@@ -47,21 +47,6 @@ constexpr int kXcds = 8;
 
 // Byte of 16-byte piece g of row r in a 64-byte-pitch LDS tile.
 __device__ inline int swz(int r, int g) { return r * 64 + ((g ^ ((r >> 1) & 3)) << 4); }
-// The upper halves of two f32 words as one bf16 pair (a low, b high).
-__device__ inline unsigned top16(float a, float b) {
-    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
-}
-__device__ inline float cut(float v) { return __uint_as_float(__float_as_uint(v) & 0xFFFF0000u); }
-
-// quant (nibble - 8) of the nibble at bit p <= 12 of w, exactly: the nibble
-// placed in the significand of 2^(23 - p) counts units of 1.
-template <int P>
-__device__ inline float quant(unsigned w) {
-    constexpr unsigned one = (unsigned)(127 + 23 - P) << 23;
-    constexpr float base = (float)(1u << (23 - P)) + 8.0f;
-    return __uint_as_float((w & (0xFu << P)) | one) - base;
-}
-
 template <int BM, int BN, int WM, int WN, int WK, int KB, int PD, bool GG>
 __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q4_0_gemm(
     const float *__restrict__ x, int M, int K, const uint8_t *__restrict__ w, int N, int n_mt,
@@ -149,33 +134,33 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
             float md[4], lo[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                md[e] = v[e] - cut(v[e]);
-                lo[e] = md[e] - cut(md[e]);
+                md[e] = v[e] - q4_cut(v[e]);
+                lo[e] = md[e] - q4_cut(md[e]);
             }
             char *p = buf + a_dst[i];
-            *reinterpret_cast<uint2 *>(p) = uint2{top16(v[0], v[1]), top16(v[2], v[3])};
+            *reinterpret_cast<uint2 *>(p) = uint2{q4_top16(v[0], v[1]), q4_top16(v[2], v[3])};
             *reinterpret_cast<uint2 *>(p + BM * 64) =
-                uint2{top16(md[0], md[1]), top16(md[2], md[3])};
+                uint2{q4_top16(md[0], md[1]), q4_top16(md[2], md[3])};
             *reinterpret_cast<uint2 *>(p + 2 * BM * 64) =
-                uint2{top16(lo[0], lo[1]), top16(lo[2], lo[3])};
+                uint2{q4_top16(lo[0], lo[1]), q4_top16(lo[2], lo[3])};
         }
 #pragma unroll
         for (int i = 0; i < LB; ++i) {
             if (UB % NT && t + NT * i >= UB) continue;
-            const unsigned q = r.b[i], h = r.b[i] >> 16;
-            const float e0 = quant<0>(q), e1 = quant<4>(q), e2 = quant<8>(q), e3 = quant<12>(q);
-            const float e4 = quant<0>(h), e5 = quant<4>(h), e6 = quant<8>(h), e7 = quant<12>(h);
+            float lo[4], hi[4];
+            q4_quants(r.b[i], lo, hi);
             char *p = buf + b_dst[i];
             if constexpr (GG) {  // low nibbles: elements 4g ..; high: 16 + 4g ..
-                *reinterpret_cast<uint2 *>(p) = uint2{top16(e0, e2), top16(e4, e6)};
+                *reinterpret_cast<uint2 *>(p) = uint2{q4_top16(lo[0], lo[1]), q4_top16(lo[2], lo[3])};
                 // piece g / 2 + 2: the swizzle's other half
                 const int n = (min(t + NT * i, UB - 1) >> 2) / KB;
                 const int g = t & 3;
                 *reinterpret_cast<uint2 *>(p + swz(n, (g >> 1) + 2) - swz(n, g >> 1)) =
-                    uint2{top16(e1, e3), top16(e5, e7)};
+                    uint2{q4_top16(hi[0], hi[1]), q4_top16(hi[2], hi[3])};
             } else {
                 *reinterpret_cast<u4 *>(p) =
-                    u4{top16(e0, e1), top16(e2, e3), top16(e4, e5), top16(e6, e7)};
+                    u4{q4_top16(lo[0], hi[0]), q4_top16(lo[1], hi[1]),
+                       q4_top16(lo[2], hi[2]), q4_top16(lo[3], hi[3])};
             }
         }
 #pragma unroll
@@ -434,13 +419,11 @@ mri_status launch_gemm(const float *x, size_t m, size_t k, const uint8_t *w, siz
 
 }  // namespace
 
-bool q4_gemm_supported(size_t m, size_t k, size_t n) {
-    constexpr size_t lim = 1u << 30;
-    return k >= 32 && k <= lim && m <= lim && n <= lim && (m + 63) / 16 * ((n + 15) / 16) <= lim;
-}
-
 mri_status launch_q4_gemm(const float *x, size_t m, size_t k, const uint8_t *w, size_t n_out,
                           bool ggml_order, float *out, hipStream_t s) {
+    constexpr size_t lim = INT_MAX - 512;
+    if (m > lim || k > lim || n_out > lim)
+        return set_error(MRI_ERR_UNSUPPORTED, "matmul_q4_0_dequant: a dimension past 2^31");
     return ggml_order ? launch_gemm<true>(x, m, k, w, n_out, out, s)
                       : launch_gemm<false>(x, m, k, w, n_out, out, s);
 }

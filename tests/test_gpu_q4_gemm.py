@@ -1,6 +1,7 @@
-"""matmul_q4_0_dequant on the matrix cores (more than 4 rows): every tile
-size and K split of its dispatch at the edges of their ranges, in both nibble
-orders, from weights at 2-byte alignment, against the product in 64 bits.
+"""matmul_q4_0_dequant on the matrix cores: the per-block kernel of up to 4
+rows and every tile size and K split of the tiled one, at the edges of their
+ranges, in both nibble orders, from weights at 2-byte alignment, against the
+product in 64 bits.
 
 Tolerance: the activations are split exactly and every product is exact, so
 the f32 sums alone round: the entry point's contract (1e-5 of
@@ -42,6 +43,9 @@ def check(got, x, raw, n, k):
 
 
 @pytest.mark.parametrize("m,n,k", [
+    (1, 33, 96), (2, 16, 32), (2, 40, 1056), (3, 50, 544), (4, 25, 4128),  # per block
+    (1, 70, 8224), (3, 31, 8192), (1, 20, 32768),      # 16 waves; past its LDS
+    (3, 6200, 64),                                     # tiled from 3 rows on
     (5, 1, 32), (16, 17, 288), (7, 6200, 544),          # 16-row tiles, narrow and wide
     (17, 33, 32), (32, 31, 288), (18, 8300, 320),       # 32-row tiles
     (33, 129, 96), (64, 127, 1056), (65, 300, 2048),    # 64 x 128 and its K split
