@@ -8,6 +8,8 @@
 //   q       = clamp(round_half_away(v * inv), -127, 127) as i8, NaN -> 0
 // The library is compiled with -ffp-contract=off and correctly rounded
 // f32 division, so each operation rounds exactly once, as in Rust.
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace mri {
@@ -15,6 +17,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kMaxPartials = 1024;
+constexpr int kTensorThreads = 1024;
 
 __device__ inline int8_t round_clamp_i8(float y) {
     float r = roundf(y);              // ties away from zero, like f32::round
@@ -64,40 +67,6 @@ __global__ __launch_bounds__(kThreads) void k_absmax_partial(
     if (threadIdx.x == 0) partials[blockIdx.x] = m;
 }
 
-// Quantize [m,k] with the per-tensor scale reduced from `partials`.
-// q_pad: [m][ld] (ld >= k, zero padded; chunk-permuted when perm) or null;
-// q_plain: [m*k] row-major or null.
-__global__ __launch_bounds__(kThreads) void k_quantize_tensor(
-    const float *__restrict__ x, size_t m, size_t k, size_t ld, int perm,
-    const float *__restrict__ partials, int n_partials,
-    int8_t *__restrict__ q_pad, int8_t *__restrict__ q_plain,
-    float *__restrict__ scale_out) {
-    __shared__ float red[kThreads / 64];
-    float mx = 0.0f;
-    for (int i = threadIdx.x; i < n_partials; i += blockDim.x)
-        mx = fmaxf(mx, partials[i]);
-    mx = block_max(mx, red);
-    const float scale = scale_of(mx);
-    const float inv = __fdiv_rn(1.0f, scale);
-    if (blockIdx.x == 0 && threadIdx.x == 0 && scale_out) *scale_out = scale;
-    const size_t total = m * ld;
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-         e += stride) {
-        const size_t r = e / ld, kk = e - r * ld;
-        int8_t q = 0;
-        if (kk < k) {
-            q = round_clamp_i8(x[r * k + kk] * inv);
-            if (q_plain) q_plain[r * k + kk] = q;
-        }
-        if (q_pad) {
-            size_t pos = kk;
-            if (perm) pos = (kk & ~(size_t)63) + q8_perm((int)(kk & 63));
-            q_pad[r * ld + pos] = q;
-        }
-    }
-}
-
 __device__ inline float absmax4(float m, const float4 &v) {
     return fmaxf(fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
 }
@@ -112,6 +81,68 @@ __device__ inline size_t row_pos(size_t kk, int perm) {
 // in the expression of the prefill SwiGLU kernel (k_swiglu_rows4), so that
 // the values are its own.
 __device__ inline float swiglu_elem(float g, float u) { return g / (1.0f + expf(-g)) * u; }
+
+// quantize_symmetric of [m][k] with one scale: blockIdx.y a row, the threads
+// of blockIdx.x its elements, four at a time (VEC: float4 rows and 4-byte
+// aligned int8 rows) or one.  q_pad: [m][ld] (ld >= k, zero padded;
+// chunk-permuted when perm) or null; q_plain: [m*k] row-major or null.
+// n_partials > 0: the maximum comes from k_absmax_partial; 0: every workgroup
+// reads the whole tensor (n elements) for it, which saves that launch.
+template <bool VEC>
+__global__ __launch_bounds__(kTensorThreads) void k_quantize_tensor(
+    const float *__restrict__ x, size_t n, size_t k, size_t ld, int perm,
+    const float *__restrict__ partials, int n_partials,
+    int8_t *__restrict__ q_pad, int8_t *__restrict__ q_plain,
+    float *__restrict__ scale_out) {
+    __shared__ float red[kTensorThreads / 64];
+    const size_t t = threadIdx.x;
+    float mx = 0.0f;
+    if (n_partials > 0) {
+        for (int i = (int)t; i < n_partials; i += kTensorThreads) mx = fmaxf(mx, partials[i]);
+    } else if (VEC) {
+        const float4 *x4 = reinterpret_cast<const float4 *>(x);
+        constexpr int D = 8;  // loads in flight a thread
+        for (size_t i = t; i < n / 4; i += D * kTensorThreads) {
+            float4 v[D];
+#pragma unroll
+            for (int u = 0; u < D; ++u)  // past the end: the last one again
+                v[u] = x4[min(i + u * kTensorThreads, n / 4 - 1)];
+#pragma unroll
+            for (int u = 0; u < D; ++u) mx = absmax4(mx, v[u]);
+        }
+    } else {
+        for (size_t i = t; i < n; i += kTensorThreads) mx = fmaxf(mx, fabsf(x[i]));
+    }
+    mx = block_max(mx, red);
+    const float scale = scale_of(mx);
+    const float inv = __fdiv_rn(1.0f, scale);
+    if (blockIdx.x == 0 && blockIdx.y == 0 && t == 0 && scale_out) *scale_out = scale;
+    const size_t r = blockIdx.y;
+    const float *row = x + r * k;
+    constexpr size_t W = VEC ? 4 : 1;
+    const size_t step = (size_t)gridDim.x * kTensorThreads * W;
+    for (size_t kk = (blockIdx.x * (size_t)kTensorThreads + t) * W; kk < ld; kk += step) {
+        if constexpr (VEC) {
+            int packed = 0;
+            if (kk < k) {
+                const float4 v = *reinterpret_cast<const float4 *>(row + kk);
+                packed = ((int)round_clamp_i8(v.x * inv) & 255) |
+                         (((int)round_clamp_i8(v.y * inv) & 255) << 8) |
+                         (((int)round_clamp_i8(v.z * inv) & 255) << 16) |
+                         ((int)round_clamp_i8(v.w * inv) << 24);
+                if (q_plain) *reinterpret_cast<int *>(q_plain + r * k + kk) = packed;
+            }
+            if (q_pad) *reinterpret_cast<int *>(q_pad + r * ld + row_pos(kk, perm)) = packed;
+        } else {
+            int8_t q = 0;
+            if (kk < k) {
+                q = round_clamp_i8(row[kk] * inv);
+                if (q_plain) q_plain[r * k + kk] = q;
+            }
+            if (q_pad) q_pad[r * ld + row_pos(kk, perm)] = q;
+        }
+    }
+}
 
 // One block per row: quantize_symmetric of each row separately.  NV > 0:
 // the row (16-byte aligned, k % 4 == 0, k <= NV * 4 * kThreads, 4-byte
@@ -367,6 +398,12 @@ inline int grid_for(size_t n, int per_thread = 1) {
 
 }  // namespace
 
+// Up to here every workgroup reads the whole tensor for its maximum (us a
+// matmul_int8_from_f32 to 4096 channels, against a launch for the maximum:
+// 3 x 1000 -> 777 6.7 and 8.1, 12 x 4096 10.6 and 11.2, 16 x 4096 -> 11008
+// 16.5 and 16.9; 20 x 4096 12.8 and 12.5, 60 x 4096 -> 11008 31.4 and 26.6).
+constexpr size_t kOnePassElems = 65536;
+
 size_t quantize_partials_count(size_t n) {
     size_t g = (n + (size_t)kThreads * 16 - 1) / ((size_t)kThreads * 16);
     if (g < 1) g = 1;
@@ -380,14 +417,30 @@ mri_status launch_quantize_tensor(const float *x, size_t m, size_t k,
                                   float *scale, float *partials,
                                   hipStream_t s) {
     const size_t n = m * k;
-    const int g = (int)quantize_partials_count(n);
-    hipLaunchKernelGGL(k_absmax_partial, dim3(g), dim3(kThreads), 0, s, x, n,
-                       partials);
-    MRI_LAUNCHED("k_absmax_partial");
-    hipLaunchKernelGGL(k_quantize_tensor, dim3(grid_for(m * (q_pad ? ld_out : k), 4)),
-                       dim3(kThreads), 0, s, x, m, k, q_pad ? ld_out : k,
-                       q8_perm_layout ? 1 : 0, partials, g, q_pad, q_plain,
-                       scale);
+    size_t ld = q_pad ? ld_out : k;
+    if (m == 0) {  // no rows: the scale alone (1)
+        m = 1;
+        k = ld = 0;
+    }
+    if (m > 65535) return set_error(MRI_ERR_UNSUPPORTED, "quantize: more than 65535 rows");
+    int g = 0;
+    if (n > kOnePassElems) {
+        g = (int)quantize_partials_count(n);
+        hipLaunchKernelGGL(k_absmax_partial, dim3(g), dim3(kThreads), 0, s, x, n, partials);
+        MRI_LAUNCHED("k_absmax_partial");
+    }
+    const bool vec = k % 4 == 0 && ld % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
+                     (reinterpret_cast<uintptr_t>(q_pad) & 3) == 0 &&
+                     (reinterpret_cast<uintptr_t>(q_plain) & 3) == 0;
+    const size_t per = (size_t)kTensorThreads * (vec ? 4 : 1);
+    const size_t gx = std::min<size_t>(std::max<size_t>((ld + per - 1) / per, 1), 4096);
+    const dim3 grid((unsigned)gx, (unsigned)m);
+    if (vec)
+        hipLaunchKernelGGL(k_quantize_tensor<true>, grid, dim3(kTensorThreads), 0, s, x, n, k, ld,
+                           q8_perm_layout ? 1 : 0, partials, g, q_pad, q_plain, scale);
+    else
+        hipLaunchKernelGGL(k_quantize_tensor<false>, grid, dim3(kTensorThreads), 0, s, x, n, k,
+                           ld, q8_perm_layout ? 1 : 0, partials, g, q_pad, q_plain, scale);
     MRI_LAUNCHED("k_quantize_tensor");
     return MRI_OK;
 }

@@ -1,9 +1,9 @@
-// skinny.hip — decode-shaped (5..32 rows per launch; larger M loops over
-// 32-row slices) quantized matmul on CDNA4 MFMA.
+// skinny.hip — decode-shaped (INT8: 5..63 rows; Q8_0 and W4A8: 5..32 rows per
+// launch, and prefill sizes below the LDS-tiled GEMM's) quantized matmul on
+// CDNA4 MFMA.
 //
 // The weight stream dominates (M*K activation bytes vs N*K weight bytes), so
-// both kernels stream the 1 KiB weight chunks of one 16-row tile per wave
-// (INT8: slab-major chunks; Q8_0: the tile's lap blocks, quants and scales
+// both kernels stream the 1 KiB weight chunks of 16-row tiles (INT8: slab-major chunks; Q8_0: the tile's lap blocks, quants and scales
 // together), with the activation rows read from a quantized [M][kp] buffer:
 //   * per-channel INT8: v_mfma_i32_16x16x64_i8 accumulates exact int32 dot
 //     products for 16 (m) x 16 (n) outputs; the f32 epilogue
@@ -25,20 +25,34 @@ using namespace gemv;
 namespace {
 
 // ---------------------------------------------------------------------------
-// Per-channel INT8.  MT activation tiles of 16 rows; NI = output registers
-// per lane that can hold a valid row (M <= 4 uses only lane group 0).
+// Per-channel INT8.  A workgroup takes NT tiles of 16 channels and all rows
+// (MT activation tiles of 16); its S waves split K into contiguous runs of
+// chunks, each in two register buffers of U chunks, and add their int32 sums
+// through LDS (exact in any order), each wave finishing its share of the
+// output registers.  One wave a tile, as this kernel had before, left 256
+// tiles with one wave a CU and re-read the weights for every 32 rows:
+// 24 x 4096 x 4096 8.4 -> 5.4 us, 60 x 4096 x 11008 with its quantization
+// 43.4 -> 25.5.
 // ---------------------------------------------------------------------------
-template <int MT, int NI, int U>
-__global__ __launch_bounds__(kWave) void k_skinny_int8(
+template <int MT, int NT, int U, int S>
+__global__ __launch_bounds__(S * kWave) void k_skinny_int8(
     const int8_t *__restrict__ act, int M, size_t kp,
     const float *__restrict__ sa_ptr, int sa_stride, float sa_value,
-    const v4i *__restrict__ tiles, const float *__restrict__ wscales, int N,
+    const v4i *__restrict__ tiles, const float *__restrict__ wscales, int N, int n_tiles,
     int P, float *__restrict__ out, int32_t *__restrict__ acc_out) {
-    const int T = blockIdx.x;
-    const int l = threadIdx.x;
+    constexpr int E = MT * NT * 4;  // output registers
+    extern __shared__ int32_t red[];  // [S][E][kWave]
+    const int T0 = blockIdx.x * NT;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l = threadIdx.x & 63;
     const int r = l & 15, g = l >> 4;
-    const size_t pitch = (size_t)gridDim.x * kWave;  // slab-major chunks
-    const v4i *wp = tiles + (size_t)T * kWave + l;
+    const int lo = split_lo(P, S, wv), hi = split_lo(P, S, wv + 1);
+    const int last = hi > 0 ? hi - 1 : 0;             // loads past the run re-read its end
+    const size_t pitch = (size_t)n_tiles * kWave;    // slab-major chunks
+    const v4i *wp[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)  // tiles past the end read the last (not stored)
+        wp[t] = tiles + (size_t)min(T0 + t, n_tiles - 1) * kWave + l;
     const v4i *ap[MT];
     bool aval[MT];
 #pragma unroll
@@ -48,86 +62,87 @@ __global__ __launch_bounds__(kWave) void k_skinny_int8(
         ap[mt] = reinterpret_cast<const v4i *>(act + (size_t)(aval[mt] ? m : 0) * kp) + g;
     }
     const v4i zero = {0, 0, 0, 0};
-    v4i acc[MT];
+    v4i acc[MT][NT];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[mt] = zero;
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[mt][t] = zero;
 
-    v4i wb[2][U];
+    v4i wb[2][NT][U];
     v4i ab[2][MT][U];
 
-    // Weight loads are unconditional (the chunk index is clamped to the last
-    // one) and rows m >= M are zeroed at use, so the compiler never has to
-    // wait for an older load before a conditional write to the same registers.
-    auto load_w = [&](int buf, int p0) __attribute__((always_inline)) {
+    // Loads are unconditional (the chunk index is clamped) and rows m >= M
+    // are zeroed at use, so the compiler never has to wait for an older load
+    // before a conditional write to the same registers.
+    auto load = [&](int buf, int p0) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            wb[buf][u] = __builtin_nontemporal_load(wp + (size_t)min(p0 + u, P - 1) * pitch);
-    };
-    auto load_a = [&](int buf, int p0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+                wb[buf][t][u] =
+                    __builtin_nontemporal_load(wp[t] + (size_t)min(p0 + u, last) * pitch);
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
-                ab[buf][mt][u] = ap[mt][(size_t)min(p0 + u, P - 1) * 4];
+                ab[buf][mt][u] = ap[mt][(size_t)min(p0 + u, last) * 4];
     };
-    // GUARD: only the last groups can run past P.
+    // GUARD: only the last group can run past the end.
     auto compute = [&](int buf, int p0, auto guard) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (!decltype(guard)::value || p0 + u < P) {
+            if (!decltype(guard)::value || p0 + u < hi) {
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
                     const v4i a = aval[mt] ? ab[buf][mt][u] : zero;
-                    acc[mt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, wb[buf][u], acc[mt],
-                                                                    0, 0, 0);
+#pragma unroll
+                    for (int t = 0; t < NT; ++t)
+                        acc[mt][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                            a, wb[buf][t][u], acc[mt][t], 0, 0, 0);
                 }
             }
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
 
-    load_w(0, 0);
-    load_a(0, 0);
-
     // Two register buffers: while one group of U chunks is consumed the next
-    // group's loads are in flight.  sched_barrier keeps the phases in this
-    // order so the waits before each compute phase stay partial.
-    const int p_full = P - P % (2 * U);
-    int p0 = 0;
-    for (; p0 < p_full; p0 += 2 * U) {
-        load_w(1, p0 + U);
-        load_a(1, p0 + U);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(0, p0, std::false_type{});
-        __builtin_amdgcn_sched_barrier(0);
-        load_w(0, p0 + 2 * U);
-        load_a(0, p0 + 2 * U);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(1, p0 + U, std::false_type{});
-        __builtin_amdgcn_sched_barrier(0);
+    // group's loads are in flight.
+    int p = lo;
+    load(0, p);
+    for (;;) {
+        if (p + U >= hi) {
+            compute(0, p, std::true_type{});
+            break;
+        }
+        load(1, p + U);
+        compute(0, p, std::false_type{});
+        p += U;
+        if (p + U >= hi) {
+            compute(1, p, std::true_type{});
+            break;
+        }
+        load(0, p + U);
+        compute(1, p, std::false_type{});
+        p += U;
     }
-    if (p0 < P) {
-        load_w(1, p0 + U);
-        load_a(1, p0 + U);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(0, p0, std::true_type{});
-        compute(1, p0 + U, std::true_type{});
-    }
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+        red[(wv * E + e) * kWave + l] = acc[e / 4 / NT][e / 4 % NT][e % 4];
+    __syncthreads();
 
-    const int n = T * 16 + r;
-    if (n >= N) return;
-    const float sw = wscales[n];
+    for (int e = wv; e < E; e += S) {  // register e % 4 of row tile e / 4 / NT
+        uint32_t sum = 0;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int m = mt * 16 + 4 * g + i;
-            if (m < M) {
-                const float sa = sa_ptr ? sa_ptr[(size_t)m * sa_stride] : sa_value;
-                float v = (float)acc[mt][i] * sa;
-                v = v * sw;
-                out[(size_t)m * N + n] = v;
-                if (acc_out) acc_out[(size_t)m * N + n] = acc[mt][i];
-            }
+        for (int q = 0; q < S; ++q) sum += (uint32_t)red[(q * E + e) * kWave + l];
+        const int m = e / (4 * NT) * 16 + 4 * g + (e & 3);
+        const int n = (T0 + e / 4 % NT) * 16 + r;
+        if (m < M && n < N) {
+            const float sa = sa_ptr ? sa_ptr[(size_t)m * sa_stride] : sa_value;
+            float v = (float)(int32_t)sum * sa;
+            v = v * wscales[n];
+            out[(size_t)m * N + n] = v;
+            if (acc_out) acc_out[(size_t)m * N + n] = (int32_t)sum;
         }
     }
 }
@@ -334,22 +349,41 @@ __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
     }
 }
 
-constexpr int kU = 8;
-
 // Prefill-sized M (one launch, ceil(M/32) waves per tile group): tiles per
 // wave and laps in flight (measured on MI355X at M = 64 .. 2048: two tiles
 // per wave run 1.4-1.5x faster than one; four are slower than two).
 constexpr int kPrefillNT = 2;
 constexpr int kPrefillRL = 2;
 
-template <int MT, int NI, int U>
-void launch_i8(const int8_t *act, size_t m, size_t kp, const float *sa_ptr,
+template <int MT, int NT, int U, int S>
+mri_status launch_i8(const int8_t *act, size_t m, size_t kp, const float *sa_ptr,
                int sa_stride, float sa_value, const QMatrixDev &w, float *out,
                int32_t *acc_out, hipStream_t s) {
-    hipLaunchKernelGGL((k_skinny_int8<MT, NI, U>), dim3((unsigned)w.n_tiles),
-                       dim3(kWave), 0, s, act, (int)m, kp, sa_ptr, sa_stride,
+    constexpr int lds = S * MT * NT * 4 * kWave * 4;
+    static_assert(lds <= 64 * 1024, "the waves' sums");
+    hipLaunchKernelGGL((k_skinny_int8<MT, NT, U, S>), dim3((unsigned)((w.n_tiles + NT - 1) / NT)),
+                       dim3(S * kWave), lds, s, act, (int)m, kp, sa_ptr, sa_stride,
                        sa_value, reinterpret_cast<const v4i *>(w.tiles), w.scales,
-                       (int)w.n_out, (int)(w.kp / kChunkK), out, acc_out);
+                       (int)w.n_out, (int)w.n_tiles, (int)(w.kp / kChunkK), out, acc_out);
+    MRI_LAUNCHED("k_skinny_int8");
+    return MRI_OK;
+}
+// Tiles and waves of a workgroup.  From 512 tiles, four tiles share each
+// activation load: the tiles' reads of the rows from L2 are what bounds the
+// kernel there (60 x 4096 x 11008: 35.3 us one tile each, 25.5 four).  Below,
+// one tile and as many waves as K has work for (24 x 4096 x 4096 with its
+// quantization: 15.4 us one wave, 13.3 four, 12.5 sixteen; 12 x 512 x 2048: 6.4
+// four, 7.6 sixteen).
+template <int MT>
+mri_status launch_i8_rows(const int8_t *act, size_t m, size_t kp, const float *sa_ptr,
+                          int sa_stride, float sa_value, const QMatrixDev &w, float *out,
+                          int32_t *acc_out, hipStream_t s) {
+    const size_t chunks = w.kp / kChunkK;
+    if (w.n_tiles >= 512)
+        return launch_i8<MT, 4, 4, 4>(act, m, kp, sa_ptr, sa_stride, sa_value, w, out, acc_out, s);
+    if (chunks >= 48)
+        return launch_i8<MT, 1, 2, 16>(act, m, kp, sa_ptr, sa_stride, sa_value, w, out, acc_out, s);
+    return launch_i8<MT, 1, 4, 4>(act, m, kp, sa_ptr, sa_stride, sa_value, w, out, acc_out, s);
 }
 
 // AG activation groups per wave, ns waves per tile (AG * ns groups of 16 rows).
@@ -384,15 +418,17 @@ mri_status launch_skinny_int8(const int8_t *act, size_t m, const float *sa_ptr,
                               int32_t *acc_out, hipStream_t s) {
     if (w.n_tiles == 0 || m == 0) return MRI_OK;
     const size_t kp = w.kp;
-    for (size_t m0 = 0; m0 < m; m0 += 32) {
-        const size_t mc = m - m0 < 32 ? m - m0 : 32;
+    for (size_t m0 = 0; m0 < m; m0 += 64) {
+        const size_t mc = m - m0 < 64 ? m - m0 : 64;
         const int8_t *a = act + m0 * kp;
         const float *sp = sa_ptr ? sa_ptr + m0 * (size_t)sa_stride : nullptr;
         float *o = out + m0 * w.n_out;
         int32_t *ao = acc_out ? acc_out + m0 * w.n_out : nullptr;
-        if (mc <= 16) launch_i8<1, 4, kU>(a, mc, kp, sp, sa_stride, sa_value, w, o, ao, s);
-        else launch_i8<2, 4, kU>(a, mc, kp, sp, sa_stride, sa_value, w, o, ao, s);
-        MRI_LAUNCHED("k_skinny_int8");
+        const mri_status st =
+            mc <= 16   ? launch_i8_rows<1>(a, mc, kp, sp, sa_stride, sa_value, w, o, ao, s)
+            : mc <= 32 ? launch_i8_rows<2>(a, mc, kp, sp, sa_stride, sa_value, w, o, ao, s)
+                       : launch_i8_rows<4>(a, mc, kp, sp, sa_stride, sa_value, w, o, ao, s);
+        if (st) return st;
     }
     return MRI_OK;
 }
