@@ -183,10 +183,11 @@ mri_status run_int8(const int8_t *act, size_t m, const float *sa_ptr,
     return launch_skinny_int8(act, m, sa_ptr, sa_stride, sa_value, w, out, acc_out, s);
 }
 
-// matmul_q8_0_direct dispatch on quantized rows [m][kp] (chunk-permuted).
+// matmul_q8_0_direct dispatch on quantized rows (chunk-permuted), [m][kp] or
+// in mg > 0 row groups.
 mri_status run_q8(const int8_t *act, size_t m, const float *sa_rows,
                          const Q8MatrixDev &w, float *out, int32_t *block_dots,
-                         hipStream_t s, bool may_alloc) {
+                         hipStream_t s, size_t mg, bool may_alloc) {
     if (gemv_q8_supported(false, m, w.n_tiles, w.k_in, w.kp))
         return launch_gemv_q8_0(nullptr, act, m, sa_rows, w, out, block_dots, nullptr, s);
     // prefill sizes: the LDS-tiled kernel (it has no block-dot output)
@@ -197,9 +198,9 @@ mri_status run_q8(const int8_t *act, size_t m, const float *sa_rows,
             const mri_status st = gemm_ws_get(s, wsb, &ws);
             if (st) return st;
         }
-        return launch_gemm_q8_0(act, m, sa_rows, w, out, ws, s);
+        return launch_gemm_q8_0(act, m, sa_rows, w, out, ws, s, mg);
     }
-    return launch_skinny_q8_0(act, m, sa_rows, w, out, block_dots, s);
+    return launch_skinny_q8_0(act, m, sa_rows, w, out, block_dots, s, mg);
 }
 
 // Returns act rows with pitch w.kp: the caller's buffer when it already has
@@ -842,7 +843,11 @@ static mri_status matmul_blocks(const char *name, const float *input, const size
         return launch_gemv_q8_0(input, nullptr, m, nullptr, d, out, block_dots_out,
                                 act_scales_out, s);
     Carver cv;
-    const size_t o_act = cv.take(m * d.kp);
+    size_t mg = act_groups(m);
+    // the fixed staging may hold the rows but not whole groups of 16
+    if (fixed && round_up(act_bytes(m, d.kp), 256) + m * sizeof(float) > MRI_NOALLOC_SCRATCH_BYTES)
+        mg = 0;
+    const size_t o_act = cv.take(mg ? act_bytes(m, d.kp) : m * d.kp);
     const size_t o_sc = cv.take(m * sizeof(float));
     void *base = nullptr;
     if (fixed) {
@@ -859,11 +864,11 @@ static mri_status matmul_blocks(const char *name, const float *input, const size
     auto *b = static_cast<uint8_t *>(base);
     int8_t *act = reinterpret_cast<int8_t *>(b + o_act);
     float *sc = act_scales_out ? act_scales_out : reinterpret_cast<float *>(b + o_sc);
-    st = launch_quantize_rows(input, m, k, d.kp, true, act, nullptr, sc, s);
+    st = launch_quantize_rows(input, m, k, d.kp, true, act, nullptr, sc, s, mg);
     if (st) return st;
     if (d.n_out == 0) return MRI_OK;
-    if (exact) return launch_skinny_q8_0(act, m, sc, d, out, block_dots_out, s);
-    return run_q8(act, m, sc, d, out, block_dots_out, s, !fixed);
+    if (exact) return launch_skinny_q8_0(act, m, sc, d, out, block_dots_out, s, mg);
+    return run_q8(act, m, sc, d, out, block_dots_out, s, mg, !fixed);
 }
 
 extern "C" {

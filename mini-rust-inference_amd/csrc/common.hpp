@@ -45,6 +45,14 @@
 //    bytes of each chunk are permuted to match the weight chunk:
 //    element kk of a chunk sits at q8_perm(kk).
 //
+//  * From 5 rows, Q8_0 activations are in row groups instead: group a =
+//    m / 16, chunk p = k / 64; fragment (p, a) is 1 KiB at byte offset
+//    (p * MG + a) * 1024 with MG = ceil(M / 16), and holds 16-byte piece g of
+//    row m's permuted chunk at (16 g + m % 16) * 16, so that a fragment is
+//    the A operand of 16 rows x 64 k in lane order: one contiguous load
+//    where the rows give 16 segments of 64 bytes.  Rows past M hold anything
+//    (their outputs are not stored).
+//
 //  * Activations of the prefill GEMM (M >= kGemmMinRows) are packed into
 //    its MFMA fragment layout: row group g = m / 32, K step p = k / 64,
 //    half h = (k % 64) / 32; fragment (p, g, h) is 1 KiB at byte offset
@@ -81,6 +89,19 @@ inline size_t round_up(size_t v, size_t m) { return (v + m - 1) / m * m; }
 // 64-byte activation chunk: [g = 0..3][h = 0..1][8 bytes].
 __host__ __device__ inline int q8_perm(int kk) {
     return ((kk >> 3) & 3) * 16 + (kk >> 5) * 8 + (kk & 7);
+}
+
+// Row groups of the activations' row-group layout, and its bytes.
+inline size_t act_groups(size_t m) { return m > 4 ? (m + 15) / 16 : 0; }
+inline size_t act_bytes(size_t m, size_t kp) {
+    return m > 4 ? act_groups(m) * 16 * kp : m * kp;
+}
+// Byte of element kk (kk % 4 == 0 keeps 4 elements contiguous) of row r: in
+// rows of pitch ld, chunk-permuted when perm, or (mg > 0) in row groups.
+__host__ __device__ inline size_t act_pos(size_t r, size_t kk, size_t ld, int perm, size_t mg) {
+    const size_t pos = perm ? (size_t)q8_perm((int)(kk & 63)) : (kk & 63);
+    if (mg == 0) return r * ld + (kk & ~(size_t)63) + pos;
+    return (((kk >> 6) * mg + (r >> 4)) * 64 + (pos >> 4) * 16 + (r & 15)) * 16 + (pos & 15);
 }
 
 struct QMatrixDev {
@@ -184,15 +205,16 @@ mri_status launch_quantize_tensor(const float *x, size_t m, size_t k,
                                   int8_t *q_pad, int8_t *q_plain,
                                   float *scale, float *partials,
                                   hipStream_t s);
+// mg > 0: q_pad in the row-group layout (act_groups) instead of rows.
 mri_status launch_quantize_rows(const float *x, size_t m, size_t k,
                                 size_t ld_out, bool q8_perm_layout,
                                 int8_t *q_pad, int8_t *q_plain,
-                                float *scales, hipStream_t s);
+                                float *scales, hipStream_t s, size_t mg = 0);
 // The same for rows of 2k, [gate | up]: quantizes their SwiGLU, silu(g) * u
 // (the values the prefill SwiGLU kernel writes), into q_pad [m][ld_out].
 mri_status launch_swiglu_quantize_rows(const float *gu, size_t m, size_t k, size_t ld_out,
                                        bool q8_perm_layout, int8_t *q_pad, float *scales,
-                                       hipStream_t s);
+                                       hipStream_t s, size_t mg = 0);
 mri_status launch_quantize_per_channel(const float *w, size_t n, size_t k,
                                        int8_t *data, float *scales,
                                        hipStream_t s);
@@ -226,8 +248,8 @@ mri_status launch_repack_q8_0(const uint8_t *raw, Q8MatrixDev &w,
 mri_status launch_repack_q4_0(const uint8_t *raw, bool ggml_order, Q8MatrixDev &w,
                               hipStream_t s);
 
-// skinny.hip: M <= 32 rows per launch (larger M loops), one wave per tile.
-// act: [M][kp] int8 (Q8_0: chunk-permuted).  Activation scale of row m is
+// skinny.hip: M <= 64 (INT8) rows per launch (larger M loops).
+// act: [M][kp] int8 (Q8_0: chunk-permuted; mg > 0: in row groups).  Activation scale of row m is
 // sa_ptr[m * sa_stride] when sa_ptr != nullptr, else sa_value.
 mri_status launch_skinny_int8(const int8_t *act, size_t m, const float *sa_ptr,
                               int sa_stride, float sa_value,
@@ -236,7 +258,7 @@ mri_status launch_skinny_int8(const int8_t *act, size_t m, const float *sa_ptr,
 mri_status launch_skinny_q8_0(const int8_t *act, size_t m,
                               const float *sa_ptr, const Q8MatrixDev &w,
                               float *out, int32_t *block_dots,
-                              hipStream_t s);
+                              hipStream_t s, size_t mg);
 // gemv.hip: M <= 4, K split over S waves per 16-row tile, weights streamed
 // through a per-wave ring of loads.  Activations come either as one f32 row
 // x (quantized in the kernel; requires gemv_fusable, M == 1; optional
@@ -336,7 +358,8 @@ constexpr int kGemmWsCounters = 65536;
 bool gemm_q8_supported(size_t m, const Q8MatrixDev &w);
 size_t gemm_q8_ws_bytes(size_t m, const Q8MatrixDev &w);
 mri_status launch_gemm_q8_0(const int8_t *act, size_t m, const float *sa_rows,
-                            const Q8MatrixDev &w, float *out, void *ws, hipStream_t s);
+                            const Q8MatrixDev &w, float *out, void *ws, hipStream_t s,
+                            size_t mg);
 // rows: act_packed is the caller's row-major [m][k] int8 (gemm_rows_ok).
 mri_status launch_gemm_int8(const int8_t *act_packed, size_t m, const float *sa_ptr,
                             int sa_stride, float sa_value, const QMatrixDev &w,
@@ -385,8 +408,8 @@ mri_status launch_rmsnorm_stats(int mode, const float *x, const float *delta,
                                 const float *w, float eps, float *stats, hipStream_t s);
 // Quantize the normalized rows w * (x * rms_inv) from those statistics:
 // form 0 per-tensor scale into the GEMM-packed layout (ld = kp), form 1
-// per-tensor into [rows][ld] plain, form 2 per-row scales into [rows][ld]
-// chunk-permuted (Q8_0), form 3 the f32 normalized rows into `normed`.
+// per-tensor into [rows][ld] plain, form 2 per-row scales, chunk-permuted
+// (Q8_0) and in row groups as act_groups(rows) says, form 3 the f32 normalized rows into `normed`.
 mri_status launch_norm_quant(int form, const float *x, const float *w, const float *stats,
                              size_t rows, size_t d, size_t ld, int8_t *q, float *scales,
                              float *normed, hipStream_t s);
@@ -397,7 +420,8 @@ mri_status run_int8(const int8_t *act, size_t m, const float *sa_ptr, int sa_str
                     hipStream_t s);
 // may_alloc false: no workspace is allocated (no K split in the GEMM).
 mri_status run_q8(const int8_t *act, size_t m, const float *sa_rows, const Q8MatrixDev &w,
-                  float *out, int32_t *block_dots, hipStream_t s, bool may_alloc = true);
+                  float *out, int32_t *block_dots, hipStream_t s, size_t mg,
+                  bool may_alloc = true);
 mri_status launch_add_rmsnorm(float *x, const float *delta, size_t rows, size_t d,
                               const float *w, float eps, float *out, hipStream_t s);
 // RoPE of q in place; rotated k and v rows into the cache at start_pos + s.

@@ -16,7 +16,7 @@
 // kernel twice as fast as keeping that order would be.
 //
 // Operands.  Both are used in the layouts the decode kernels read:
-//   * activations: rows [M][kp] (kp = K padded to 256) with each 64-byte
+//   * activations: row groups (or rows [M][kp], kp = K padded to 256) with each 64-byte
 //     chunk permuted so that lane group g's 16 bytes are [block 2p, k 8g..+8 |
 //     block 2p+1, k 8g..+8], i.e. the 8-byte A operands of
 //     v_mfma_i32_16x16x32_i8 for both blocks of the chunk;
@@ -149,7 +149,7 @@ template <int BM, int BN, int WM, int WN, int NS, bool W4>
 __global__ __launch_bounds__(WM * WN * kQWave) void k_gemm_q8_0(
     const int8_t *__restrict__ act, int M, int kp, const float *__restrict__ sa_rows,
     const int8_t *__restrict__ laps, int N, int n_tiles, int G, int n_mt, int n_total, int ks,
-    float *__restrict__ out, float *__restrict__ part, int *__restrict__ cnt) {
+    float *__restrict__ out, float *__restrict__ part, int *__restrict__ cnt, int mg) {
     constexpr int NW = WM * WN;
     constexpr int RG = BM / 32 / WM, TT = BN / 32 / WN;  // 32 x 32 sub-tiles per wave
     constexpr int FA = BM / 8, FB = q8_b_slots<BN, NW, W4>(), FS = q8_scale_slots<BN, NW>();
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(WM * WN * kQWave) void k_gemm_q8_0(
     // region: weight tile f / 2, chunk f % 2; tiles past the end read the
     // last.  Scales: tile wv + NW * j (waves past the tile count: the last
     // tile, into a slot nothing reads), 4 bytes per lane (its 256 bytes).
-    // Step s adds 128 s bytes to an activation source, and lap s / 2 (plus
+    // Step s adds 128 s bytes (in row groups, 2 mg KiB s) to an activation source, and lap s / 2 (plus
     // 2 KiB for the second half) to a weight source.
     const int8_t *a_src[LA];
     const int8_t *b_src[LB];
@@ -196,8 +196,11 @@ __global__ __launch_bounds__(WM * WN * kQWave) void k_gemm_q8_0(
     for (int j = 0; j < LA; ++j) {
         const int f = wv + NW * j;
         const int row = min(BM * mt + 16 * (f >> 1) + (l & 15), M - 1);
-        a_src[j] = act + (size_t)row * kp + 64 * (f & 1) + 16 * (l >> 4);
+        const int grp = min(BM / 16 * mt + (f >> 1), mg - 1);
+        a_src[j] = mg ? act + ((size_t)(f & 1) * mg + grp) * 1024 + 16 * l
+                      : act + (size_t)row * kp + 64 * (f & 1) + 16 * (l >> 4);
     }
+    const size_t a_step = mg ? (size_t)mg * 2048 : 128;
 #pragma unroll
     for (int j = 0; j < LB; ++j) {
         const int f = wv + NW * j;
@@ -219,7 +222,7 @@ __global__ __launch_bounds__(WM * WN * kQWave) void k_gemm_q8_0(
     auto issue = [&](int s) __attribute__((always_inline)) {
         const int sc = min(s, s1 - 1);
         const unsigned base = lds0 + (unsigned)((s % NS) * STAGE);
-        const size_t ao = (size_t)sc * 128;
+        const size_t ao = (size_t)sc * a_step;
         const size_t bo = (size_t)(sc >> 1) * lap_bytes + (size_t)(sc & 1) * (W4 ? 1024 : 2048);
         const size_t so = (size_t)(sc >> 1) * lap_bytes;
 #pragma unroll
@@ -467,7 +470,7 @@ int q8_ks(size_t m, const Q8MatrixDev &w) {
 
 template <int BM, int BN, int WM, int WN, int NS, bool W4>
 mri_status launch_q8_inst(const int8_t *act, size_t m, const float *sa_rows,
-                          const Q8MatrixDev &w, float *out, void *ws, hipStream_t s) {
+                          const Q8MatrixDev &w, float *out, void *ws, hipStream_t s, int mg) {
     constexpr size_t lds = (size_t)NS * q8_stage_bytes<BM, BN, WM * WN, W4>();
     static DeviceOnce attr;
     MRI_HIP(attr.run([&](int) {
@@ -485,7 +488,7 @@ mri_status launch_q8_inst(const int8_t *act, size_t m, const float *sa_rows,
     hipLaunchKernelGGL((k_gemm_q8_0<BM, BN, WM, WN, NS, W4>), dim3((unsigned)grid),
                        dim3(WM * WN * kQWave), lds, s, act, (int)m, (int)w.kp, sa_rows, w.laps,
                        (int)w.n_out, (int)w.n_tiles, (int)w.laps_per_tile(), (int)n_mt,
-                       (int)total, ks, out, part, cnt);
+                       (int)total, ks, out, part, cnt, mg);
     MRI_LAUNCHED("k_gemm_q8_0");
     return MRI_OK;
 }
@@ -507,8 +510,8 @@ bool gemm_q8_supported(size_t m, const Q8MatrixDev &w) {
            m * w.n_out < (1ull << 31);
 }
 
-// act: quantized rows [m][w.kp], chunk-permuted (launch_quantize_rows with
-// the Q8_0 layout); sa_rows: their scales.
+// act: quantized rows, chunk-permuted (launch_quantize_rows with the Q8_0
+// layout), [m][w.kp] or in mg > 0 row groups; sa_rows: their scales.
 // Tiles of 128 rows x 64 channels, 8 waves of 32 x 32, two LDS stages
 // (about 52 KiB; the 126 VGPRs hold two workgroups per CU, four waves per
 // SIMD, either way).  Three stages took 1-2 % longer (M = 512, K = 4096:
@@ -521,9 +524,11 @@ bool gemm_q8_supported(size_t m, const Q8MatrixDev &w) {
 // than 4 of 64 x 32 halve each wave's serial fold per step and took the
 // latency floor from 43 to 39 us (512 x 11008 -> 4096: 108 against 117).
 mri_status launch_gemm_q8_0(const int8_t *act, size_t m, const float *sa_rows,
-                            const Q8MatrixDev &w, float *out, void *ws, hipStream_t s) {
-    if (w.w4) return launch_q8_inst<kQ8BM, kQ8BN, 4, 2, 2, true>(act, m, sa_rows, w, out, ws, s);
-    return launch_q8_inst<kQ8BM, kQ8BN, 4, 2, 2, false>(act, m, sa_rows, w, out, ws, s);
+                            const Q8MatrixDev &w, float *out, void *ws, hipStream_t s,
+                            size_t mg) {
+    if (w.w4)
+        return launch_q8_inst<kQ8BM, kQ8BN, 4, 2, 2, true>(act, m, sa_rows, w, out, ws, s, (int)mg);
+    return launch_q8_inst<kQ8BM, kQ8BN, 4, 2, 2, false>(act, m, sa_rows, w, out, ws, s, (int)mg);
 }
 
 // [tile counters (kGemmWsCounters ints, shared with the INT8 GEMM's)]

@@ -252,7 +252,7 @@ mri_status proj_normed(mri_llama *m, const mri_weight_ref &w, size_t rows, float
                                         : handle_dev(static_cast<const mri_q4_0_matrix *>(w.ptr));
         if (dv.n_out == 0) return MRI_OK;
         TRY(prepare(2, dv.kp));
-        return run_q8(m->qact, rows, m->qscale, dv, out, nullptr, s);
+        return run_q8(m->qact, rows, m->qscale, dv, out, nullptr, s, act_groups(rows));
     }
     default:
         TRY(prepare(3, d));
@@ -472,9 +472,9 @@ mri_status block(mri_llama *m, size_t li, size_t rows, size_t start, mri_kv_cach
             return set_error(MRI_ERR_SHAPE_MISMATCH, "down projection: k_in != ffn_dim");
         if (dv.n_out) {
             TRY(launch_swiglu_quantize_rows(m->gu, rows, g.ffn_dim, dv.kp, true, m->qact,
-                                            m->qscale, s));
+                                            m->qscale, s, act_groups(rows)));
             m->qform = -1;  // qact no longer holds the normalized rows
-            TRY(run_q8(m->qact, rows, m->qscale, dv, m->tmp, nullptr, s));
+            TRY(run_q8(m->qact, rows, m->qscale, dv, m->tmp, nullptr, s, act_groups(rows)));
         }
         return out_tail(next_norm);
     }

@@ -71,12 +71,6 @@ __device__ inline float absmax4(float m, const float4 &v) {
     return fmaxf(fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
 }
 
-// Offset of element kk (kk % 4 == 0 keeps 4 elements contiguous) in a
-// padded output row, chunk-permuted when perm.
-__device__ inline size_t row_pos(size_t kk, int perm) {
-    return perm ? (kk & ~(size_t)63) + q8_perm((int)(kk & 63)) : kk;
-}
-
 // SwiGLU of one element, silu(g) * u (activation/swiglu.rs, silu.rs:23-26),
 // in the expression of the prefill SwiGLU kernel (k_swiglu_rows4), so that
 // the values are its own.
@@ -132,14 +126,14 @@ __global__ __launch_bounds__(kTensorThreads) void k_quantize_tensor(
                          ((int)round_clamp_i8(v.w * inv) << 24);
                 if (q_plain) *reinterpret_cast<int *>(q_plain + r * k + kk) = packed;
             }
-            if (q_pad) *reinterpret_cast<int *>(q_pad + r * ld + row_pos(kk, perm)) = packed;
+            if (q_pad) *reinterpret_cast<int *>(q_pad + act_pos(r, kk, ld, perm, 0)) = packed;
         } else {
             int8_t q = 0;
             if (kk < k) {
                 q = round_clamp_i8(row[kk] * inv);
                 if (q_plain) q_plain[r * k + kk] = q;
             }
-            if (q_pad) q_pad[r * ld + row_pos(kk, perm)] = q;
+            if (q_pad) q_pad[act_pos(r, kk, ld, perm, 0)] = q;
         }
     }
 }
@@ -155,7 +149,7 @@ template <int NV, bool GLU = false, int TH = kThreads>
 __global__ __launch_bounds__(TH) void k_quantize_rows(
     const float *__restrict__ x, size_t k, size_t ld, int perm,
     int8_t *__restrict__ q_pad, int8_t *__restrict__ q_plain,
-    float *__restrict__ scales) {
+    float *__restrict__ scales, size_t mg) {
     __shared__ float red[TH / 64];
     const size_t r = blockIdx.x;
     const float *row = x + r * (GLU ? 2 * k : k);
@@ -206,13 +200,13 @@ __global__ __launch_bounds__(TH) void k_quantize_rows(
                                    (((int)round_clamp_i8(v[j].z * inv) & 255) << 16) |
                                    ((int)round_clamp_i8(v[j].w * inv) << 24);
                 if (q_plain) *reinterpret_cast<int *>(q_plain + r * k + kk) = packed;
-                if (q_pad) *reinterpret_cast<int *>(q_pad + r * ld + row_pos(kk, perm)) = packed;
+                if (q_pad) *reinterpret_cast<int *>(q_pad + act_pos(r, kk, ld, perm, mg)) = packed;
             }
         }
         // zero padding of the output row
         if (q_pad)
             for (size_t kk = k + 4 * t; kk < ld; kk += 4 * TH)
-                *reinterpret_cast<int *>(q_pad + r * ld + row_pos(kk, perm)) = 0;
+                *reinterpret_cast<int *>(q_pad + act_pos(r, kk, ld, perm, mg)) = 0;
     } else {
         auto elem = [&](size_t i) { return GLU ? swiglu_elem(row[i], urow[i]) : row[i]; };
         for (size_t i = t; i < k; i += blockDim.x) mx = fmaxf(mx, fabsf(elem(i)));
@@ -226,7 +220,7 @@ __global__ __launch_bounds__(TH) void k_quantize_rows(
                 q = round_clamp_i8(elem(kk) * inv);
                 if (q_plain) q_plain[r * k + kk] = q;
             }
-            if (q_pad) q_pad[r * ld + row_pos(kk, perm)] = q;
+            if (q_pad) q_pad[act_pos(r, kk, ld, perm, mg)] = q;
         }
     }
 }
@@ -251,16 +245,17 @@ inline int rows_nv(const float *x, size_t k, size_t ld, const int8_t *q_pad,
 // the same bytes; from 128 rows up 1024 threads gave the same times).
 template <bool GLU, int TH = GLU ? 1024 : kThreads>
 void launch_rows(const float *x, size_t m, size_t k, size_t ld, int perm, int8_t *q_pad,
-                 int8_t *q_plain, float *scales, hipStream_t s) {
+                 int8_t *q_plain, float *scales, hipStream_t s, size_t mg = 0) {
     if constexpr (!GLU && TH == kThreads) {
-        if (m <= 32) return launch_rows<false, 1024>(x, m, k, ld, perm, q_pad, q_plain, scales, s);
+        if (m <= 32)
+            return launch_rows<false, 1024>(x, m, k, ld, perm, q_pad, q_plain, scales, s, mg);
     }
     const dim3 grid((unsigned)m), block(TH);
     switch (rows_nv(x, k, ld, q_pad, q_plain, TH)) {
-    case 4: hipLaunchKernelGGL((k_quantize_rows<4, GLU, TH>), grid, block, 0, s, x, k, ld, perm, q_pad, q_plain, scales); break;
-    case 8: hipLaunchKernelGGL((k_quantize_rows<8, GLU, TH>), grid, block, 0, s, x, k, ld, perm, q_pad, q_plain, scales); break;
-    case 16: hipLaunchKernelGGL((k_quantize_rows<16, GLU, TH>), grid, block, 0, s, x, k, ld, perm, q_pad, q_plain, scales); break;
-    default: hipLaunchKernelGGL((k_quantize_rows<0, GLU, TH>), grid, block, 0, s, x, k, ld, perm, q_pad, q_plain, scales); break;
+    case 4: hipLaunchKernelGGL((k_quantize_rows<4, GLU, TH>), grid, block, 0, s, x, k, ld, perm, q_pad, q_plain, scales, mg); break;
+    case 8: hipLaunchKernelGGL((k_quantize_rows<8, GLU, TH>), grid, block, 0, s, x, k, ld, perm, q_pad, q_plain, scales, mg); break;
+    case 16: hipLaunchKernelGGL((k_quantize_rows<16, GLU, TH>), grid, block, 0, s, x, k, ld, perm, q_pad, q_plain, scales, mg); break;
+    default: hipLaunchKernelGGL((k_quantize_rows<0, GLU, TH>), grid, block, 0, s, x, k, ld, perm, q_pad, q_plain, scales, mg); break;
     }
 }
 
@@ -469,7 +464,7 @@ namespace {
 // all rows, as matmul_int8_from_f32 quantizes its input), GEMM-packed
 // layout, grid over the rows padded to 32 (padding rows are zero); FORM 1:
 // per-tensor, [rows][ld] plain; FORM 2: per-row scales (matmul_q8_0_direct),
-// [rows][ld] chunk-permuted; FORM 3: the normalized f32 rows themselves.
+// chunk-permuted, rows or (mg > 0) row groups; FORM 3: the normalized f32 rows themselves.
 // The quantized values equal those of quantizing the stored normalized
 // rows: the same y, the same max, the same scale.
 template <int NV, int FORM>
@@ -528,13 +523,13 @@ __global__ __launch_bounds__(kThreads) void k_norm_quant(
                                (((int)round_clamp_i8(y[c].z * inv) & 255) << 16) |
                                ((int)round_clamp_i8(y[c].w * inv) << 24);
             const size_t pos = FORM == 0 ? gemm_pack_offset(r, kk, mg)
-                                         : (size_t)r * ld + row_pos(kk, FORM == 2);
+                                         : act_pos(r, kk, ld, FORM == 2, FORM == 2 ? mg : 0);
             *reinterpret_cast<int *>(q + pos) = packed;
         }
     }
     for (size_t kk = (size_t)d + 4 * t; kk < ld; kk += 4 * kThreads) {  // zero padding
         const size_t pos = FORM == 0 ? gemm_pack_offset(r, kk, mg)
-                                     : (size_t)r * ld + row_pos(kk, FORM == 2);
+                                     : act_pos(r, kk, ld, FORM == 2, FORM == 2 ? mg : 0);
         *reinterpret_cast<int *>(q + pos) = 0;
     }
 }
@@ -547,7 +542,7 @@ mri_status launch_norm_quant(int form, const float *x, const float *w, const flo
     if (!rows) return MRI_OK;
     if (d % 4 || d > 8192 || (form != 3 && (ld < d || ld % 4)))
         return set_error(MRI_ERR_INVALID_ARGUMENT, "norm quant: unsupported row shape");
-    const size_t mg = gemm_row_groups(rows);
+    const size_t mg = form == 0 ? gemm_row_groups(rows) : act_groups(rows);
     const dim3 g((unsigned)(form == 0 ? mg * 32 : rows)), b(kThreads);
     auto go = [&](auto nv) {
         constexpr int NV = decltype(nv)::value;
@@ -578,19 +573,19 @@ mri_status launch_pack_gemm(const int8_t *src, size_t m, size_t k, size_t ld, si
 mri_status launch_quantize_rows(const float *x, size_t m, size_t k,
                                 size_t ld_out, bool q8_perm_layout,
                                 int8_t *q_pad, int8_t *q_plain,
-                                float *scales, hipStream_t s) {
+                                float *scales, hipStream_t s, size_t mg) {
     if (m == 0) return MRI_OK;
     launch_rows<false>(x, m, k, q_pad ? ld_out : k, q8_perm_layout ? 1 : 0, q_pad, q_plain,
-                       scales, s);
+                       scales, s, mg);
     MRI_LAUNCHED("k_quantize_rows");
     return MRI_OK;
 }
 
 mri_status launch_swiglu_quantize_rows(const float *gu, size_t m, size_t k, size_t ld_out,
                                        bool q8_perm_layout, int8_t *q_pad, float *scales,
-                                       hipStream_t s) {
+                                       hipStream_t s, size_t mg) {
     if (m == 0) return MRI_OK;
-    launch_rows<true>(gu, m, k, ld_out, q8_perm_layout ? 1 : 0, q_pad, nullptr, scales, s);
+    launch_rows<true>(gu, m, k, ld_out, q8_perm_layout ? 1 : 0, q_pad, nullptr, scales, s, mg);
     MRI_LAUNCHED("k_quantize_rows(swiglu)");
     return MRI_OK;
 }

@@ -3,8 +3,10 @@
 // CDNA4 MFMA.
 //
 // The weight stream dominates (M*K activation bytes vs N*K weight bytes), so
-// both kernels stream the 1 KiB weight chunks of 16-row tiles (INT8: slab-major chunks; Q8_0: the tile's lap blocks, quants and scales
-// together), with the activation rows read from a quantized [M][kp] buffer:
+// both kernels stream the 1 KiB weight chunks of 16-row tiles
+// (INT8: slab-major chunks; Q8_0: the tile's lap blocks, quants and scales
+// together), with the activation rows read from a quantized buffer ([M][kp], or
+// row groups):
 //   * per-channel INT8: v_mfma_i32_16x16x64_i8 accumulates exact int32 dot
 //     products for 16 (m) x 16 (n) outputs; the f32 epilogue
 //     ((f32)acc * s_a) * s_w runs once at the end (int8.rs:93);
@@ -16,6 +18,7 @@
 // (activation) m = 4*(l/16) + i and column (weight row) n = l % 16.
 // The M <= 4 decode case uses the K-split kernels of gemv_int8.hip and
 // gemv_q8.hip instead.
+#include <algorithm>
 #include <type_traits>
 
 #include "gemv_common.hpp"
@@ -148,7 +151,7 @@ __global__ __launch_bounds__(S * kWave) void k_skinny_int8(
 }
 
 // ---------------------------------------------------------------------------
-// Q8_0, up to 32 rows: AG groups of 16 activation rows.  One wave per tile
+// Q8_0: AG groups of 16 activation rows a wave.  One wave per tile
 // of 16 output channels sweeps all of K in laps of one scale group (4
 // chunks = 8 blocks) and keeps RL laps of loads in flight: per chunk one
 // 16-byte load of the weight chunk and, per activation group, one 16-byte
@@ -167,71 +170,63 @@ __global__ __launch_bounds__(S * kWave) void k_skinny_int8(
 // 2(c % 2) + h of piece c / 2 with each nibble moved to the high half of its
 // byte (16 * quant as int8), and the MFMA result is divided by 16 exactly.
 // ---------------------------------------------------------------------------
-template <int AG, int NT, int TPW, int RL, bool DEBUG, bool W4>
+template <int AG, int TPW, int RL, bool DEBUG, bool W4>
 __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
     const int8_t *__restrict__ act, int M, int kp, const float *__restrict__ sa_rows,
     const v4i *__restrict__ laps, int N, int n_tiles, int G, int nb, float *__restrict__ out,
-    int32_t *__restrict__ block_dots, int ns) {
-    // wave -> (group of NT adjacent tiles, set of AG activation groups); the
-    // ns waves of a tile group are adjacent, so they share a workgroup (or
-    // neighbouring ones) and the weight chunks they all stream are fetched
-    // from HBM once.  NT > 1 spreads each activation load over NT tiles.
-    // With several workgroups per tile group the grid (a multiple of 8) is
+    int32_t *__restrict__ block_dots, int ns, int mg) {
+    // wave -> (tile, set of AG activation groups); the ns waves of a tile are
+    // adjacent, so they share a workgroup (or neighbouring ones) and the weight
+    // chunks they all stream are fetched from HBM once.
+    // With several workgroups per tile the grid (a multiple of 8) is
     // taken XCD-major: workgroups are dispatched to the 8 XCDs round-robin,
     // and consecutive indices of one XCD share its L2.
     int blk = blockIdx.x;
     if (ns > TPW) blk = (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8);
     const int wv = blk * TPW + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int TG = wv / ns;
-    const int a0 = (wv - TG * ns) * AG;  // first activation group of the wave
-    if (TG * NT >= n_tiles) return;  // whole waves only; the kernel has no barrier
+    const int T = wv / ns;
+    const int a0 = (wv - T * ns) * AG;  // first activation group of the wave
+    if (T >= n_tiles) return;  // whole waves only; the kernel has no barrier
     const int l = threadIdx.x & 63;
     const int r = l & 15, g = l >> 4;
-    // the tiles' lap blocks: quant piece c of lap q at v4i offset
-    // q * LB + c * 64 (+ lane), the lap's scales at q * LB + SO (+ row);
-    // tiles past the end read the last tile and store nothing
+    // the tile's lap blocks: quant piece c of lap q at v4i offset
+    // q * LB + c * 64 (+ lane), the lap's scales at q * LB + SO (+ row)
     constexpr size_t LB = (W4 ? kQ4LapBytes : kQ8LapBytes) / 16;
     constexpr int SO = W4 ? 128 : 256;
     constexpr int NP = W4 ? 2 : 4;  // quant pieces per lap and lane
-    const v4i *wp[NT];
-    const v4i *sp[NT];
-    int n[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        const int T = min(TG * NT + t, n_tiles - 1);
-        wp[t] = laps + (size_t)T * G * LB + l;
-        sp[t] = laps + (size_t)T * G * LB + SO + r;
-        n[t] = TG * NT + t < n_tiles ? (TG * NT + t) * 16 + r : N;
-    }
+    const v4i *wp = laps + (size_t)T * G * LB + l;
+    const v4i *sp = laps + (size_t)T * G * LB + SO + r;
+    const int n = T * 16 + r;
+    // the activations: this lane's 16 bytes of chunk p of its rows at
+    // ap[a][p * cs], in rows (past M: row 0) or in mg row groups
     const v4i *ap[AG];
-    float sa[AG][4], fs[AG][NT][4];
+    const size_t cs = mg ? (size_t)mg * 64 : 4;
+    float sa[AG][4], fs[AG][4];
 #pragma unroll
     for (int a = 0; a < AG; ++a) {
         const int m = 16 * (a0 + a) + r;
-        ap[a] = reinterpret_cast<const v4i *>(act + (size_t)(m < M ? m : 0) * kp) + g;
+        const v4i *av = reinterpret_cast<const v4i *>(act);
+        ap[a] = mg ? av + 64 * min(a0 + a, mg - 1) + l
+                   : av + (size_t)(m < M ? m : 0) * (kp / 16) + g;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             sa[a][i] = sa_rows[min(16 * (a0 + a) + 4 * g + i, M - 1)];
-#pragma unroll
-            for (int t = 0; t < NT; ++t) fs[a][t][i] = 0.0f;
+            fs[a][i] = 0.0f;
         }
     }
-    v4i wr[RL][NT][4];
+    v4i wr[RL][4];
     v4i xr[RL][4][AG];
-    v4i sr[RL][NT];
+    v4i sr[RL];
 #pragma unroll
     for (int u = 0; u < RL; ++u) {
         const int q = min(u, G - 1);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
+            if (c < NP) wr[u][c] = __builtin_nontemporal_load(wp + (size_t)q * LB + c * 64);
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
-                if (c < NP) wr[u][t][c] = __builtin_nontemporal_load(wp[t] + (size_t)q * LB + c * 64);
-#pragma unroll
-            for (int a = 0; a < AG; ++a) xr[u][c][a] = ap[a][(size_t)(4 * q + c) * 4];
+            for (int a = 0; a < AG; ++a) xr[u][c][a] = ap[a][(size_t)(4 * q + c) * cs];
         }
-#pragma unroll
-        for (int t = 0; t < NT; ++t) sr[u][t] = sp[t][(size_t)q * LB];
+        sr[u] = sp[(size_t)q * LB];
     }
     const v4i zero = {0, 0, 0, 0};
     // Without W4 each block's MFMA starts from the bits of 1.5 * 2^23, so an
@@ -246,29 +241,26 @@ __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
         constexpr int U = decltype(slot)::value;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            v4i d[2][AG][NT];
+            v4i d[2][AG];
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
+                long bv;
+                if constexpr (W4) {
+                    const v4i pc = wr[U][c >> 1];
+                    const int wd = (c & 1) ? (h ? pc.w : pc.z) : (h ? pc.y : pc.x);
+                    constexpr int kHi = (int)0xF0F0F0F0u;
+                    bv = (long)(((unsigned long)(unsigned)(wd & kHi) << 32) |
+                                (unsigned)((wd << 4) & kHi));
+                } else {
+                    bv = h ? hi8(wr[U][c]) : lo8(wr[U][c]);
+                }
 #pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    long bv;
+                for (int a = 0; a < AG; ++a) {
+                    d[h][a] = __builtin_amdgcn_mfma_i32_16x16x32_i8(
+                        h ? hi8(xr[U][c][a]) : lo8(xr[U][c][a]), bv, cinit, 0, 0, 0);
                     if constexpr (W4) {
-                        const v4i pc = wr[U][t][c >> 1];
-                        const int wd = (c & 1) ? (h ? pc.w : pc.z) : (h ? pc.y : pc.x);
-                        constexpr int kHi = (int)0xF0F0F0F0u;
-                        bv = (long)(((unsigned long)(unsigned)(wd & kHi) << 32) |
-                                    (unsigned)((wd << 4) & kHi));
-                    } else {
-                        bv = h ? hi8(wr[U][t][c]) : lo8(wr[U][t][c]);
-                    }
 #pragma unroll
-                    for (int a = 0; a < AG; ++a) {
-                        d[h][a][t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(
-                            h ? hi8(xr[U][c][a]) : lo8(xr[U][c][a]), bv, cinit, 0, 0, 0);
-                        if constexpr (W4) {
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) d[h][a][t][i] >>= 4;
-                        }
+                        for (int i = 0; i < 4; ++i) d[h][a][i] >>= 4;
                     }
                 }
             }
@@ -276,50 +268,42 @@ __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
                 const size_t p = (size_t)(4 * (L + RL) + c);
                 if (!W4 || (c & 1)) {
                     const int pi = W4 ? c >> 1 : c;
-#pragma unroll
-                    for (int t = 0; t < NT; ++t)
-                        wr[U][t][pi] =
-                            __builtin_nontemporal_load(wp[t] + (size_t)(L + RL) * LB + pi * 64);
+                    wr[U][pi] =
+                        __builtin_nontemporal_load(wp + (size_t)(L + RL) * LB + pi * 64);
                 }
 #pragma unroll
-                for (int a = 0; a < AG; ++a) xr[U][c][a] = ap[a][p * 4];
+                for (int a = 0; a < AG; ++a) xr[U][c][a] = ap[a][p * cs];
             }
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int b = 8 * L + 2 * c + h;
                 if (!decltype(check)::value || b < nb) {
+                    const unsigned word = (unsigned)sr[U][c];
+                    const float ds = f16_bits_to_f32(h ? (word >> 16) : (word & 0xFFFFu));
 #pragma unroll
-                    for (int t = 0; t < NT; ++t) {
-                        const unsigned word = (unsigned)sr[U][t][c];
-                        const float ds = f16_bits_to_f32(h ? (word >> 16) : (word & 0xFFFFu));
+                    for (int a = 0; a < AG; ++a) {
 #pragma unroll
-                        for (int a = 0; a < AG; ++a) {
+                        for (int i = 0; i < 4; ++i) {
+                            const int dv = d[h][a][i];
+                            float tm = (W4 ? (float)dv : __int_as_float(dv) - kDotBiasF) *
+                                       sa[a][i];
+                            tm = tm * ds;
+                            fs[a][i] = fs[a][i] + tm;
+                        }
+                        if constexpr (DEBUG) {
 #pragma unroll
                             for (int i = 0; i < 4; ++i) {
-                                const int dv = d[h][a][t][i];
-                                float tm = (W4 ? (float)dv : __int_as_float(dv) - kDotBiasF) *
-                                           sa[a][i];
-                                tm = tm * ds;
-                                fs[a][t][i] = fs[a][t][i] + tm;
-                            }
-                            if constexpr (DEBUG) {
-#pragma unroll
-                                for (int i = 0; i < 4; ++i) {
-                                    const int m = 16 * (a0 + a) + 4 * g + i;
-                                    if (m < M && n[t] < N)
-                                        block_dots[((size_t)m * N + n[t]) * nb + b] =
-                                            W4 ? d[h][a][t][i] : d[h][a][t][i] - kDotBias;
-                                }
+                                const int m = 16 * (a0 + a) + 4 * g + i;
+                                if (m < M && n < N)
+                                    block_dots[((size_t)m * N + n) * nb + b] =
+                                        W4 ? d[h][a][i] : d[h][a][i] - kDotBias;
                             }
                         }
                     }
                 }
             }
         }
-        if (refill) {
-#pragma unroll
-            for (int t = 0; t < NT; ++t) sr[U][t] = sp[t][(size_t)(L + RL) * LB];
-        }
+        if (refill) sr[U] = sp[(size_t)(L + RL) * LB];
         // keep the next lap's uses of its (younger) loads below this point
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -336,29 +320,20 @@ __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
             if (u < rem) lap(k * RL + u, u, false, T1{});
         });
     }
+    if (n >= N) return;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        if (n[t] >= N) continue;
+    for (int a = 0; a < AG; ++a)
 #pragma unroll
-        for (int a = 0; a < AG; ++a)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int m = 16 * (a0 + a) + 4 * g + i;
-                if (m < M) out[(size_t)m * N + n[t]] = fs[a][t][i];
-            }
-    }
+        for (int i = 0; i < 4; ++i) {
+            const int m = 16 * (a0 + a) + 4 * g + i;
+            if (m < M) out[(size_t)m * N + n] = fs[a][i];
+        }
 }
-
-// Prefill-sized M (one launch, ceil(M/32) waves per tile group): tiles per
-// wave and laps in flight (measured on MI355X at M = 64 .. 2048: two tiles
-// per wave run 1.4-1.5x faster than one; four are slower than two).
-constexpr int kPrefillNT = 2;
-constexpr int kPrefillRL = 2;
 
 template <int MT, int NT, int U, int S>
 mri_status launch_i8(const int8_t *act, size_t m, size_t kp, const float *sa_ptr,
-               int sa_stride, float sa_value, const QMatrixDev &w, float *out,
-               int32_t *acc_out, hipStream_t s) {
+                     int sa_stride, float sa_value, const QMatrixDev &w, float *out,
+                     int32_t *acc_out, hipStream_t s) {
     constexpr int lds = S * MT * NT * 4 * kWave * 4;
     static_assert(lds <= 64 * 1024, "the waves' sums");
     hipLaunchKernelGGL((k_skinny_int8<MT, NT, U, S>), dim3((unsigned)((w.n_tiles + NT - 1) / NT)),
@@ -387,27 +362,29 @@ mri_status launch_i8_rows(const int8_t *act, size_t m, size_t kp, const float *s
 }
 
 // AG activation groups per wave, ns waves per tile (AG * ns groups of 16 rows).
-template <int AG, int NT, int TPW, int RL, bool DEBUG, bool W4>
+template <int AG, int TPW, int RL, bool DEBUG, bool W4>
 void launch_q8_w(const int8_t *act, size_t m, size_t kp, const float *sa_rows,
-                 const Q8MatrixDev &w, float *out, int32_t *block_dots, int ns, hipStream_t s) {
+                 const Q8MatrixDev &w, float *out, int32_t *block_dots, int ns, int mg,
+                 hipStream_t s) {
     const int G = (int)w.laps_per_tile();
-    const size_t waves = (w.n_tiles + NT - 1) / NT * (size_t)ns;
+    const size_t waves = w.n_tiles * (size_t)ns;
     size_t grid = (waves + TPW - 1) / TPW;
     if (ns > TPW) grid = (grid + 7) / 8 * 8;  // XCD-major mapping (whole waves past the end exit)
-    hipLaunchKernelGGL((k_skinny_q8_0<AG, NT, TPW, RL, DEBUG, W4>),
+    hipLaunchKernelGGL((k_skinny_q8_0<AG, TPW, RL, DEBUG, W4>),
                        dim3((unsigned)grid), dim3(TPW * kWave), 0, s,
                        act, (int)m, (int)kp, sa_rows, reinterpret_cast<const v4i *>(w.laps),
                        (int)w.n_out, (int)w.n_tiles, G,
-                       (int)w.n_blocks, out, block_dots, ns);
+                       (int)w.n_blocks, out, block_dots, ns, mg);
 }
 
-template <int AG, int NT, int TPW, int RL, bool DEBUG>
+template <int AG, int TPW, int RL, bool DEBUG>
 void launch_q8(const int8_t *act, size_t m, size_t kp, const float *sa_rows,
-               const Q8MatrixDev &w, float *out, int32_t *block_dots, int ns, hipStream_t s) {
+               const Q8MatrixDev &w, float *out, int32_t *block_dots, int ns, int mg,
+                 hipStream_t s) {
     if (w.w4)
-        launch_q8_w<AG, NT, TPW, RL, DEBUG, true>(act, m, kp, sa_rows, w, out, block_dots, ns, s);
+        launch_q8_w<AG, TPW, RL, DEBUG, true>(act, m, kp, sa_rows, w, out, block_dots, ns, mg, s);
     else
-        launch_q8_w<AG, NT, TPW, RL, DEBUG, false>(act, m, kp, sa_rows, w, out, block_dots, ns, s);
+        launch_q8_w<AG, TPW, RL, DEBUG, false>(act, m, kp, sa_rows, w, out, block_dots, ns, mg, s);
 }
 
 }  // namespace
@@ -433,41 +410,50 @@ mri_status launch_skinny_int8(const int8_t *act, size_t m, const float *sa_ptr,
     return MRI_OK;
 }
 
+namespace {
+
+// A wave takes AG groups of 16 rows of one tile; the ns waves of a tile share
+// a workgroup (four of them, above 32 rows) and so its weights in the CU's L1.
+// Groups a wave: two where that still leaves a wave for every SIMD (the
+// weight operand then feeds two MFMAs), else one, and one for W4, whose
+// weights cost half the bytes (us a call, two / one: Q8_0 100 x 4096 x 4096
+// 21.0 / 22.7, 100 x 4096 x 11008 43.3 / 46.8, 64 x 4096 x 4096 18.9 / 16.0,
+// 100 x 1024 x 1024 9.7 / 8.2, 32 x 4096 x 11008 20.9 / 23.5, 24 x 4096 x 4096
+// 17.6 / 13.6; W4 100 x 11008 x 4096 51.4 / 42.9, 32 x 4096 x 11008 22.0 /
+// 19.5).  With the activations in row groups (1 KiB a load) two tiles a wave,
+// which halved the row-strided loads, are no longer faster: 100 x 4096 x 4096
+// 30.9 in rows and two tiles, 21.0 now; 16 x 4096 x 11008 16.9, 15.4 now.
+template <int RL2, int RL1, bool DEBUG>
+void launch_q8_groups(const int8_t *act, size_t m, size_t kp, const float *sa_rows,
+                      const Q8MatrixDev &w, float *out, int32_t *block_dots, int mg,
+                      hipStream_t s) {
+    const int n1 = (int)((m + 15) / 16), n2 = (int)((m + 31) / 32);
+    const size_t simds = 4 * (size_t)std::max(device_cus(), 1);
+    const bool one = w.w4 || w.n_tiles * (size_t)n1 <= simds;
+    if (m <= 16)
+        launch_q8<1, 1, RL1, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, 1, mg, s);
+    else if (m <= 32 && one)
+        launch_q8<1, 2, RL1, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, 2, mg, s);
+    else if (m <= 32)
+        launch_q8<2, 1, RL2, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, 1, mg, s);
+    else if (one)
+        launch_q8<1, 4, RL2, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, n1, mg, s);
+    else
+        launch_q8<2, 4, RL2, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, n2, mg, s);
+}
+
+}  // namespace
+
 mri_status launch_skinny_q8_0(const int8_t *act, size_t m,
                               const float *sa_rows, const Q8MatrixDev &w,
                               float *out, int32_t *block_dots,
-                              hipStream_t s) {
+                              hipStream_t s, size_t mg) {
     if (w.n_tiles == 0 || m == 0) return MRI_OK;
-    const size_t kp = w.kp;
-    if (m > 32) {
-        // one launch for all rows: ceil(m/32) waves of 32 rows per weight
-        // tile, four to a workgroup; the weights stream from HBM about once
-        // instead of once per 32-row slice
-        const int ns = (int)((m + 31) / 32);
-        if (block_dots)
-            launch_q8<2, kPrefillNT, 4, kPrefillRL, true>(act, m, kp, sa_rows, w, out, block_dots, ns, s);
-        else
-            launch_q8<2, kPrefillNT, 4, kPrefillRL, false>(act, m, kp, sa_rows, w, out, block_dots, ns, s);
-        MRI_LAUNCHED("k_skinny_q8_0");
-        return MRI_OK;
-    }
-    for (size_t m0 = 0; m0 < m; m0 += 32) {
-        const size_t mc = m - m0 < 32 ? m - m0 : 32;
-        const int8_t *a = act + m0 * kp;
-        const float *sp = sa_rows + m0;
-        float *o = out + m0 * w.n_out;
-        int32_t *bd = block_dots ? block_dots + m0 * w.n_out * w.n_blocks : nullptr;
-        // one wave per tile and workgroup (measured on MI355X: splitting a
-        // tile's row groups over waves, or grouping tiles, is slower)
-        if (bd) {
-            if (mc <= 16) launch_q8<1, 1, 1, 2, true>(a, mc, kp, sp, w, o, bd, 1, s);
-            else launch_q8<2, 1, 1, 2, true>(a, mc, kp, sp, w, o, bd, 1, s);
-        } else {
-            if (mc <= 16) launch_q8<1, 1, 1, 3, false>(a, mc, kp, sp, w, o, bd, 1, s);
-            else launch_q8<2, 1, 1, 2, false>(a, mc, kp, sp, w, o, bd, 1, s);
-        }
-        MRI_LAUNCHED("k_skinny_q8_0");
-    }
+    if (block_dots)
+        launch_q8_groups<2, 2, true>(act, m, w.kp, sa_rows, w, out, block_dots, (int)mg, s);
+    else
+        launch_q8_groups<2, 3, false>(act, m, w.kp, sa_rows, w, out, nullptr, (int)mg, s);
+    MRI_LAUNCHED("k_skinny_q8_0");
     return MRI_OK;
 }
 
