@@ -759,8 +759,9 @@ mri_status mri_matmul_int8_from_f32(const float *input, const size_t *dims, size
     mri_status st = current_device(&dev);
     if (st) return st;
     auto s = static_cast<hipStream_t>(stream);
-    if (d.n_out > 0 && gemv_fusable(m, k, input) && aligned(act_q_out, 4) &&
-        gemv_int8_supported(true, m, d.n_tiles, k, d.kp))
+    if (d.n_out > 0 && aligned(act_q_out, 4) &&
+        ((gemv_fusable(m, k, input) && gemv_int8_supported(true, m, d.n_tiles, k, d.kp)) ||
+         gemv_int8_rows_fusable(m, k, d.kp, d.n_tiles, input)))
         return launch_gemv_int8(input, nullptr, m, nullptr, 0, 0.0f, d, out, act_q_out,
                                 act_scale_out, acc_out, s);
     const bool gemm = m >= kGemmMinRows;

@@ -312,6 +312,7 @@ struct RowOps {
                out2 || silu_n > 0;
     }
 };
+bool gemv_int8_rows_fusable(size_t m, size_t k, size_t kp, size_t n_tiles, const float *x);
 bool gemv_int8_supported(bool fused, size_t m, size_t n_tiles, size_t k, size_t kp);
 // The device matrices behind the public handles (capi.cpp).
 const QMatrixDev &handle_dev(const mri_qmatrix *h);

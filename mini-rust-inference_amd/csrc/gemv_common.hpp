@@ -153,6 +153,9 @@ struct ActIn {
     const unsigned long long *in_keys = nullptr;  // x is a table row picked by keys (RowOps)
     int n_in_keys = 0;
     uint32_t *tok_out = nullptr;
+    // rows > 1 of the fused path that share one scale (INT8): K is all their
+    // elements, x is contiguous, row_k a row's and row_pitch its LDS bytes
+    int row_k = 0, row_pitch = 0;
 
     ActIn(const float *x_, const int8_t *act_, int k, int8_t *aq, float *so, const RowOps &o)
         : x(x_), act(act_), K(k), act_q_out(aq), scale_out(so), norm_w(o.norm_w), eps(o.eps),
@@ -358,7 +361,8 @@ __device__ inline void act_begin(const ActIn &in, int n16, const v4i (&xr)[XR], 
 // q8_perm) or kLayMasked (masked_off, with the zero word beside each data
 // word).
 enum : int { kLayPlain = 0, kLayPerm = 1, kLayMasked = 2 };
-template <int S, int XR, bool FUSED, bool OPS>
+// ROWS: several rows with one scale (ActIn::row_k), plain layout.
+template <int S, int XR, bool FUSED, bool OPS, bool ROWS = false>
 __device__ inline void act_end(const ActIn &in, int layout, v4i (&xr)[XR], const v4i (&wn)[XR],
                                int8_t *s_act, float *red, float &scale, bool writer) {
     __syncthreads();
@@ -408,7 +412,8 @@ __device__ inline void act_end(const ActIn &in, int layout, v4i (&xr)[XR], const
                 const int kk = 4 * j;
                 const int pos = layout == kLayMasked ? masked_off(kk)
                                 : layout == kLayPerm ? (kk & ~63) + q8_perm(kk & 63)
-                                                     : kk;
+                                : ROWS ? kk / in.row_k * in.row_pitch + kk % in.row_k
+                                       : kk;
                 const int packed =
                     (q0 & 255) | ((q1 & 255) << 8) | ((q2 & 255) << 16) | (q3 << 24);
                 *reinterpret_cast<int *>(s_act + pos) = packed;

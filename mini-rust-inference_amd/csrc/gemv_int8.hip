@@ -64,7 +64,7 @@ __global__ __launch_bounds__(S * TPW * kWave) void k_gemv_int8(
     v4i wr[D];
 
     v4i xr[XR];
-    const int n16 = FUSED ? in.K / 4 : M * kp / 16;
+    const int n16 = FUSED ? in.K / 4 : M * kp / 16;  // in.K: all the rows' elements
     const float *xrow = in.x;
     if constexpr (FUSED && OPS) xrow = row_of_keys<NW>(in);  // the step's token row
     stage_load<NW, XR>(FUSED ? reinterpret_cast<const v4i *>(xrow)
@@ -101,7 +101,8 @@ __global__ __launch_bounds__(S * TPW * kWave) void k_gemv_int8(
         inv = act_end_lazy<NW, XR, OPS>(in, xr, wn, reinterpret_cast<float *>(s_act), red,
                                         sa_value, blockIdx.x == 0);
     else
-        act_end<NW, XR, FUSED, OPS>(in, kLayPlain, xr, wn, s_act, red, sa_value, blockIdx.x == 0);
+        act_end<NW, XR, FUSED, OPS, (NI > 1)>(in, kLayPlain, xr, wn, s_act, red, sa_value,
+                                              blockIdx.x == 0);
     if constexpr (FUSED) sa_ptr = nullptr;
 
     // LAZY: quantize lap L (chunks c0 + L*D ..; lane l: values 256 e + 4 l of
@@ -219,7 +220,7 @@ CfgI8 pick_i8(bool fused, size_t n_tiles, size_t m, size_t k, size_t kp, bool la
     else if (kp <= 4096) { c.s = 4; c.d = 8; }
     else { c.s = 8; c.d = 8; }
     const size_t threads = (size_t)c.s * c.tpw * kWave;
-    const size_t nx = ceil_div(fused ? k / 4 : m * kp / 16, threads);
+    const size_t nx = ceil_div(fused ? m * k / 4 : m * kp / 16, threads);
     c.xr = nx <= 4 ? 4 : nx <= 8 ? 8 : nx <= 12 ? 12 : 0;
     if (c.xr == 0 || lds_i8(c.s, c.tpw, m, kp) > kMaxLds) c.s = 0;
     if (c.s && fused && lazy_ok && m == 1 && c.tpw == 1 &&
@@ -272,6 +273,17 @@ bool gemv_int8_supported(bool fused, size_t m, size_t n_tiles, size_t k, size_t 
     return m >= 1 && m <= (size_t)kMaxM && pick_i8(fused, n_tiles, m, k, kp).s > 0;
 }
 
+// f32 rows that one launch quantizes (with their common scale) and multiplies:
+// every workgroup stages them all, as far as its registers hold them (12
+// float4 a thread).  Against the quantizer's own launch (us a call in a
+// graph, bit-identical): 3 x 1000 -> 777 4.3 and 6.6, 2 x 4096 -> 4096 7.0
+// and 9.4, 3 x 4096 -> 4096 8.3 and 9.5, 2 x 4096 -> 11008 11.1 and 13.5.
+bool gemv_int8_rows_fusable(size_t m, size_t k, size_t kp, size_t n_tiles, const float *x) {
+    return m > 1 && m <= (size_t)kMaxM && k > 0 && k % 4 == 0 && x &&
+           (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
+           pick_i8(true, n_tiles, m, k, kp).s > 0;
+}
+
 // The row operations apply to the fused path only, with aligned operands.
 bool row_ops_ok(const float *x, const RowOps &o) {
     auto al = [](const float *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
@@ -304,7 +316,15 @@ mri_status launch_gemv_int8(const float *x, const int8_t *act, size_t m,
     if (c.s == 0) return set_error(MRI_ERR_INVALID_ARGUMENT, "gemv: shape not supported");
     if (!row_ops_ok(x, ops))
         return set_error(MRI_ERR_INVALID_ARGUMENT, "gemv: row operations need the fused path");
-    const ActIn in(x, act, (int)w.k_in, act_q_out, scale_out, ops);
+    ActIn in(x, act, (int)w.k_in, act_q_out, scale_out, ops);
+    if (x && m > 1) {
+        in.row_k = (int)w.k_in;
+        in.row_pitch = (int)w.kp;
+        in.K = (int)(m * w.k_in);
+        dispatch_i8<4, true>(c, in, m, nullptr, 0, 0.0f, w, out, acc_out, st);
+        MRI_LAUNCHED("k_gemv_int8");
+        return MRI_OK;
+    }
     if (ops.any()) {
         dispatch_i8<1, true, true>(c, in, m, nullptr, 0, 0.0f, w, out, acc_out, st);
     } else if (x) {

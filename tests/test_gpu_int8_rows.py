@@ -1,5 +1,6 @@
-"""matmul_int8_from_f32 and matmul_int8_rows at 5-63 rows, bit for bit against
-the oracle: the channel counts and K at which the kernel's tiles, waves and
+"""matmul_int8_from_f32 at 2-63 rows, bit for bit against the oracle: rows
+that the decode kernel quantizes itself, at every tile count it splits by;
+the channel counts and K at which the kernel's tiles, waves and
 K runs change (1 or 4 tiles of 16 channels, 4 or 16 waves, runs of no, one
 and uneven chunks), rows in one to four tiles of 16, K with and without whole
 float4s, and the sizes on both sides of the one-pass quantization."""
@@ -13,6 +14,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("m,n,k", [
+    (2, 33, 4), (3, 777, 1000), (4, 70, 3072), (4, 16, 3076), (3, 41, 1001),  # decode
+    (2, 100, 6000), (3, 8200, 512), (4, 16400, 132), (2, 16390, 8192),
     (5, 1, 1), (16, 17, 63), (17, 40, 130), (33, 33, 1000), (63, 16, 3009),
     (20, 70, 3072), (49, 50, 4111),                      # 16 waves
     (6, 8192, 64), (31, 8177, 200), (40, 8200, 72), (63, 8193, 1028),  # four tiles
