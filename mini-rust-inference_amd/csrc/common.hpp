@@ -47,10 +47,11 @@
 //
 //  * From 5 rows, Q8_0 activations are in row groups instead: group a =
 //    m / 16, chunk p = k / 64; fragment (p, a) is 1 KiB at byte offset
-//    (p * MG + a) * 1024 with MG = ceil(M / 16), and holds 16-byte piece g of
-//    row m's permuted chunk at (16 g + m % 16) * 16, so that a fragment is
-//    the A operand of 16 rows x 64 k in lane order: one contiguous load
-//    where the rows give 16 segments of 64 bytes.  Rows past M hold anything
+//    (p * MG + a) * 1024 with MG = ceil(M / 16), and holds row m's permuted
+//    chunk at (m % 16) * 64, so that the A operand of 16 rows x 64 k is one
+//    contiguous KiB where the rows give 16 half cache lines.  (16-byte pieces
+//    in lane order read as fast, but the rows' quantizers then write 16-byte
+//    pieces of lines that other XCDs write too.)  Rows past M hold anything
 //    (their outputs are not stored).
 //
 //  * Activations of the prefill GEMM (M >= kGemmMinRows) are packed into
@@ -101,7 +102,7 @@ inline size_t act_bytes(size_t m, size_t kp) {
 __host__ __device__ inline size_t act_pos(size_t r, size_t kk, size_t ld, int perm, size_t mg) {
     const size_t pos = perm ? (size_t)q8_perm((int)(kk & 63)) : (kk & 63);
     if (mg == 0) return r * ld + (kk & ~(size_t)63) + pos;
-    return (((kk >> 6) * mg + (r >> 4)) * 64 + (pos >> 4) * 16 + (r & 15)) * 16 + (pos & 15);
+    return ((kk >> 6) * mg + (r >> 4)) * 1024 + (r & 15) * 64 + pos;
 }
 
 struct QMatrixDev {

@@ -197,8 +197,9 @@ __global__ __launch_bounds__(WM * WN * kQWave) void k_gemm_q8_0(
         const int f = wv + NW * j;
         const int row = min(BM * mt + 16 * (f >> 1) + (l & 15), M - 1);
         const int grp = min(BM / 16 * mt + (f >> 1), mg - 1);
-        a_src[j] = mg ? act + ((size_t)(f & 1) * mg + grp) * 1024 + 16 * l
-                      : act + (size_t)row * kp + 64 * (f & 1) + 16 * (l >> 4);
+        a_src[j] = (mg ? act + ((size_t)(f & 1) * mg + grp) * 1024 + 64 * (l & 15)
+                       : act + (size_t)row * kp + 64 * (f & 1)) +
+                   16 * (l >> 4);
     }
     const size_t a_step = mg ? (size_t)mg * 2048 : 128;
 #pragma unroll

@@ -170,7 +170,7 @@ __global__ __launch_bounds__(S * kWave) void k_skinny_int8(
 // 2(c % 2) + h of piece c / 2 with each nibble moved to the high half of its
 // byte (16 * quant as int8), and the MFMA result is divided by 16 exactly.
 // ---------------------------------------------------------------------------
-template <int AG, int TPW, int RL, bool DEBUG, bool W4>
+template <int AG, int TPW, int RL, int CS, bool DEBUG, bool W4>
 __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
     const int8_t *__restrict__ act, int M, int kp, const float *__restrict__ sa_rows,
     const v4i *__restrict__ laps, int N, int n_tiles, int G, int nb, float *__restrict__ out,
@@ -194,20 +194,28 @@ __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
     constexpr size_t LB = (W4 ? kQ4LapBytes : kQ8LapBytes) / 16;
     constexpr int SO = W4 ? 128 : 256;
     constexpr int NP = W4 ? 2 : 4;  // quant pieces per lap and lane
-    const v4i *wp = laps + (size_t)T * G * LB + l;
-    const v4i *sp = laps + (size_t)T * G * LB + SO + r;
+    // (addresses as a wave-uniform base and a 32-bit lane offset, so that no
+    // vector instruction goes into them: a wave that is alone on its SIMD is
+    // bound by those it issues)
+    const char *wp = reinterpret_cast<const char *>(laps + (size_t)T * G * LB);
+    const unsigned wl = 16 * l, sl = 16 * (SO + r);
+    auto at = [](const char *base, unsigned lane) __attribute__((always_inline)) {
+        return reinterpret_cast<const v4i *>(base + (size_t)lane);
+    };
     const int n = T * 16 + r;
     // the activations: this lane's 16 bytes of chunk p of its rows at
-    // ap[a][p * cs], in rows (past M: row 0) or in mg row groups
-    const v4i *ap[AG];
-    const size_t cs = mg ? (size_t)mg * 64 : 4;
+    // act + p * cs + al[a], in rows (past M: row 0) or in mg row groups.  CS
+    // states the stride for one group or rows, where it is known: a lap's four
+    // loads then share one address (14 x 12288 x 2560: 4 % of a wave's time).
+    unsigned al[AG];
+    const size_t cs = CS ? CS : mg ? (size_t)mg * 1024 : 64;
+    const char *ap = reinterpret_cast<const char *>(act);
     float sa[AG][4], fs[AG][4];
 #pragma unroll
     for (int a = 0; a < AG; ++a) {
         const int m = 16 * (a0 + a) + r;
-        const v4i *av = reinterpret_cast<const v4i *>(act);
-        ap[a] = mg ? av + 64 * min(a0 + a, mg - 1) + l
-                   : av + (size_t)(m < M ? m : 0) * (kp / 16) + g;
+        al[a] = mg ? 1024u * (unsigned)min(a0 + a, mg - 1) + 64 * r + 16 * g
+                   : (unsigned)(m < M ? m : 0) * (unsigned)kp + 16 * g;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             sa[a][i] = sa_rows[min(16 * (a0 + a) + 4 * g + i, M - 1)];
@@ -222,11 +230,12 @@ __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
         const int q = min(u, G - 1);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            if (c < NP) wr[u][c] = __builtin_nontemporal_load(wp + (size_t)q * LB + c * 64);
+            if (c < NP)
+                wr[u][c] = __builtin_nontemporal_load(at(wp + ((size_t)q * LB + c * 64) * 16, wl));
 #pragma unroll
-            for (int a = 0; a < AG; ++a) xr[u][c][a] = ap[a][(size_t)(4 * q + c) * cs];
+            for (int a = 0; a < AG; ++a) xr[u][c][a] = *at(ap + (size_t)(4 * q + c) * cs, al[a]);
         }
-        sr[u] = sp[(size_t)q * LB];
+        sr[u] = *at(wp + (size_t)q * LB * 16, sl);
     }
     const v4i zero = {0, 0, 0, 0};
     // Without W4 each block's MFMA starts from the bits of 1.5 * 2^23, so an
@@ -268,11 +277,11 @@ __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
                 const size_t p = (size_t)(4 * (L + RL) + c);
                 if (!W4 || (c & 1)) {
                     const int pi = W4 ? c >> 1 : c;
-                    wr[U][pi] =
-                        __builtin_nontemporal_load(wp + (size_t)(L + RL) * LB + pi * 64);
+                    wr[U][pi] = __builtin_nontemporal_load(
+                        at(wp + ((size_t)(L + RL) * LB + pi * 64) * 16, wl));
                 }
 #pragma unroll
-                for (int a = 0; a < AG; ++a) xr[U][c][a] = ap[a][p * cs];
+                for (int a = 0; a < AG; ++a) xr[U][c][a] = *at(ap + p * cs, al[a]);
             }
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -303,7 +312,7 @@ __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
                 }
             }
         }
-        if (refill) sr[U] = sp[(size_t)(L + RL) * LB];
+        if (refill) sr[U] = *at(wp + (size_t)(L + RL) * LB * 16, sl);
         // keep the next lap's uses of its (younger) loads below this point
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -362,7 +371,7 @@ mri_status launch_i8_rows(const int8_t *act, size_t m, size_t kp, const float *s
 }
 
 // AG activation groups per wave, ns waves per tile (AG * ns groups of 16 rows).
-template <int AG, int TPW, int RL, bool DEBUG, bool W4>
+template <int AG, int TPW, int RL, int CS, bool DEBUG, bool W4>
 void launch_q8_w(const int8_t *act, size_t m, size_t kp, const float *sa_rows,
                  const Q8MatrixDev &w, float *out, int32_t *block_dots, int ns, int mg,
                  hipStream_t s) {
@@ -370,21 +379,21 @@ void launch_q8_w(const int8_t *act, size_t m, size_t kp, const float *sa_rows,
     const size_t waves = w.n_tiles * (size_t)ns;
     size_t grid = (waves + TPW - 1) / TPW;
     if (ns > TPW) grid = (grid + 7) / 8 * 8;  // XCD-major mapping (whole waves past the end exit)
-    hipLaunchKernelGGL((k_skinny_q8_0<AG, TPW, RL, DEBUG, W4>),
+    hipLaunchKernelGGL((k_skinny_q8_0<AG, TPW, RL, CS, DEBUG, W4>),
                        dim3((unsigned)grid), dim3(TPW * kWave), 0, s,
                        act, (int)m, (int)kp, sa_rows, reinterpret_cast<const v4i *>(w.laps),
                        (int)w.n_out, (int)w.n_tiles, G,
                        (int)w.n_blocks, out, block_dots, ns, mg);
 }
 
-template <int AG, int TPW, int RL, bool DEBUG>
+template <int AG, int TPW, int RL, int CS, bool DEBUG>
 void launch_q8(const int8_t *act, size_t m, size_t kp, const float *sa_rows,
                const Q8MatrixDev &w, float *out, int32_t *block_dots, int ns, int mg,
                  hipStream_t s) {
     if (w.w4)
-        launch_q8_w<AG, TPW, RL, DEBUG, true>(act, m, kp, sa_rows, w, out, block_dots, ns, mg, s);
+        launch_q8_w<AG, TPW, RL, CS, DEBUG, true>(act, m, kp, sa_rows, w, out, block_dots, ns, mg, s);
     else
-        launch_q8_w<AG, TPW, RL, DEBUG, false>(act, m, kp, sa_rows, w, out, block_dots, ns, mg, s);
+        launch_q8_w<AG, TPW, RL, CS, DEBUG, false>(act, m, kp, sa_rows, w, out, block_dots, ns, mg, s);
 }
 
 }  // namespace
@@ -430,16 +439,18 @@ void launch_q8_groups(const int8_t *act, size_t m, size_t kp, const float *sa_ro
     const int n1 = (int)((m + 15) / 16), n2 = (int)((m + 31) / 32);
     const size_t simds = 4 * (size_t)std::max(device_cus(), 1);
     const bool one = w.w4 || w.n_tiles * (size_t)n1 <= simds;
-    if (m <= 16)
-        launch_q8<1, 1, RL1, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, 1, mg, s);
+    if (m <= 16 && mg == 1)
+        launch_q8<1, 1, RL1, 1024, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, 1, mg, s);
+    else if (m <= 16)
+        launch_q8<1, 1, RL1, 64, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, 1, mg, s);
     else if (m <= 32 && one)
-        launch_q8<1, 2, RL1, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, 2, mg, s);
+        launch_q8<1, 2, RL1, 0, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, 2, mg, s);
     else if (m <= 32)
-        launch_q8<2, 1, RL2, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, 1, mg, s);
+        launch_q8<2, 1, RL2, 0, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, 1, mg, s);
     else if (one)
-        launch_q8<1, 4, RL2, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, n1, mg, s);
+        launch_q8<1, 4, RL2, 0, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, n1, mg, s);
     else
-        launch_q8<2, 4, RL2, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, n2, mg, s);
+        launch_q8<2, 4, RL2, 0, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, n2, mg, s);
 }
 
 }  // namespace
