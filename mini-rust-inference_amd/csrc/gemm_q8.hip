@@ -26,8 +26,8 @@
 // 32 x 32); each ring stage is half a lap (4 blocks): per stage it stages
 // BM x 128 bytes of activation fragments, BN x 128 bytes of weight chunks
 // and the lap's scales in LDS by global_load_lds (16 bytes per lane, each
-// lane its own address, so a fragment of 16 rows x 64 bytes is gathered
-// straight from the row-major activations), NS stages deep: the loads of
+// lane its own address: a fragment of 16 rows x 64 bytes is one KiB of a row
+// group, or is gathered from row-major activations), NS stages deep: the loads of
 // the next stages fly while one is folded.  Each of the 8 waves (4 x 2) owns
 // 32 rows x 32 channels; two workgroups share a CU, four waves per SIMD, and
 // the MFMA results, sums and operands all stay in VGPRs.
