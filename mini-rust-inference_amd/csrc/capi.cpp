@@ -115,10 +115,12 @@ mri_status scratch_get(hipStream_t stream, size_t bytes, void **ptr) {
 }
 
 // Per-(device, stream) workspaces of the kernels that count arrivals (the
-// stream-K GEMM, the one-row argmax).  Zeroed whenever they are
-// (re)allocated; the kernels leave their counters zero after every call.
+// stream-K GEMM, the Q4_0 GEMM's K parts, the one-row argmax).  Zeroed whenever
+// they are (re)allocated; the kernels leave their counters zero after every call.
+// The Q4_0 GEMM has its own: it uses it in no captured call, so it may grow
+// beside recorded graphs, whose INT8 and Q8_0 GEMMs replay with g_ws.
 static std::mutex g_ws_mu;
-static std::map<std::pair<int, hipStream_t>, Scratch> g_ws, g_aws;
+static std::map<std::pair<int, hipStream_t>, Scratch> g_ws, g_q4ws, g_aws;
 
 static mri_status zeroed_ws_get(std::map<std::pair<int, hipStream_t>, Scratch> &map,
                                 hipStream_t stream, size_t bytes, void **ptr) {
@@ -144,6 +146,10 @@ static mri_status zeroed_ws_get(std::map<std::pair<int, hipStream_t>, Scratch> &
 
 mri_status gemm_ws_get(hipStream_t stream, size_t bytes, void **ptr) {
     return zeroed_ws_get(g_ws, stream, bytes, ptr);
+}
+
+mri_status q4_ws_get(hipStream_t stream, size_t bytes, void **ptr) {
+    return zeroed_ws_get(g_q4ws, stream, bytes, ptr);
 }
 
 mri_status argmax_ws_get(hipStream_t stream, void **ptr, size_t bytes) {

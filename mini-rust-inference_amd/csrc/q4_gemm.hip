@@ -394,8 +394,8 @@ mri_status launch_gemm(const float *x, size_t m, size_t k, const uint8_t *w, siz
             return launch_cfg<32, 32, 1, 2, 8, 8, 2, GG>(x, m, k, w, n, 1, out, nullptr, s);
         return launch_cfg<32, 64, 1, 4, 4, 4, 3, GG>(x, m, k, w, n, 1, out, nullptr, s);
     }
-    // A stream that is being captured gets no K split: its workspace may be
-    // neither allocated nor grown under a recorded graph.
+    // A stream that is being captured gets no K split: no recorded graph holds
+    // the workspace, which may therefore grow at any later call.
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     bool may_split = hipStreamIsCapturing(s, &cap) == hipSuccess;
     if (!may_split) (void)hipGetLastError();
@@ -406,7 +406,7 @@ mri_status launch_gemm(const float *x, size_t m, size_t k, const uint8_t *w, siz
     if (parts > 1) {
         const Tile &tl = kTiles[tile];
         const size_t tiles = ((m + tl.bm - 1) / tl.bm) * ((n + tl.bn - 1) / tl.bn);
-        const mri_status st = gemm_ws_get(
+        const mri_status st = q4_ws_get(
             s, kGemmWsCounters * sizeof(int) + tiles * parts * tl.bm * tl.bn * sizeof(float), &ws);
         if (st) return st;
     }

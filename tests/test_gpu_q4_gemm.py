@@ -12,7 +12,8 @@ import numpy as np
 import pytest
 
 import closed_form as CF
-from gpu_util import F32, dev, empty, host, synth_q4_0, torch
+from gpu_util import (F32, assert_bits_equal, dev, empty, host, synth_q4_0, synth_q8_0,
+                      torch)
 
 pytestmark = pytest.mark.gpu
 
@@ -116,3 +117,40 @@ def test_captured_call_needs_no_workspace():
         g.replay()
         check(host(out), x, raw, n, k)
         xd.copy_(xd * 1.0)
+
+
+def test_recorded_graph_outlives_a_larger_call():
+    """The Q8_0 GEMM's K split recorded on a stream, then a Q4_0 call on that
+    stream whose parts need more memory than it: replays and eager Q4_0 calls
+    in turn give their own results."""
+    t = torch()
+    rng = np.random.default_rng(9)
+    m, n, k = 200, 6000, 4096
+    w8 = mri().Q8Matrix.from_raw_bytes(synth_q8_0(rng, n, k), n, k)
+    x8, out8 = dev(rng.standard_normal((m, k)).astype(F32)), empty((m, n), t.float32)
+    m4, n4, k4 = 256, 11008, 4096
+    raw = synth_q4_0(rng, n4, k4)
+    x4, w4 = dev(rng.standard_normal((m4, k4)).astype(F32)), dev(raw)
+    out4 = empty((m4, n4), t.float32)
+    s = t.cuda.Stream()
+    s.wait_stream(t.cuda.current_stream())
+    with t.cuda.stream(s):
+        mri().matmul_q8_0_direct(x8, w8, out8)
+    t.cuda.synchronize()
+    want8 = host(out8)
+    g = t.cuda.CUDAGraph()
+    with t.cuda.graph(g, stream=s):
+        mri().matmul_q8_0_direct(x8, w8, out8)
+    want4 = None
+    for _ in range(3):
+        out8.zero_()
+        s.wait_stream(t.cuda.current_stream())
+        with t.cuda.stream(s):
+            mri().matmul_q4_0_dequant(x4, w4, n4, k4, out4)
+            g.replay()
+        t.cuda.synchronize()
+        assert_bits_equal(host(out8), want8, "replay")
+        if want4 is None:
+            want4 = host(out4)
+            check(want4, host(x4), raw, n4, k4)
+        assert_bits_equal(host(out4), want4, "Q4_0 beside the graph")

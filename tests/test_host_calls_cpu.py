@@ -1,0 +1,89 @@
+"""What calls do on the host, under a stand-in for the HIP runtime
+(fake_hip.c): the device memory they take and give back.  Each check runs in a
+process of its own, which loads the stand-in before the library."""
+import ctypes as C
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+X, W, OUT = 0x100000, 0x200000, 0x300000   # operands: 16-byte aligned addresses
+STREAM = 0x5000
+
+
+class Host:
+    def __init__(self, fake):
+        self.f = C.CDLL(fake, mode=C.RTLD_GLOBAL)
+        self.f.fake_launch.restype = C.c_char_p
+        self.f.fake_alloc_bytes.restype = C.c_size_t
+        sys.modules["torch"] = None   # its HIP runtime stays out of this process
+        sys.path.insert(0, os.path.join(os.path.dirname(HERE), "mini-rust-inference_amd"))
+        import mri_qmatmul
+        self.m, self.lib = mri_qmatmul, mri_qmatmul.lib()
+
+    def set(self, name, value):
+        C.c_int.in_dll(self.f, name).value = value
+
+    def live(self):
+        return {i for i in range(self.f.fake_allocs()) if self.f.fake_live(i)}
+
+    def launches(self, start=0):
+        out = []
+        for i in range(start, self.f.fake_launches()):
+            v = (C.c_uint * 6)()
+            name = self.f.fake_launch(i, v).decode()
+            out.append((name, list(v)))
+        return out
+
+    def q8_0(self, m, k, n):
+        h = C.c_void_p()
+        self.m.check(self.lib.mri_q8_0_matrix_from_raw_device(W, n * k // 32 * 34, n, k, STREAM,
+                                                              C.byref(h)))
+        return lambda: self.lib.mri_matmul_q8_0_direct(X, (C.c_size_t * 2)(m, k), 2, h, OUT,
+                                                       None, None, STREAM)
+
+    def q4_0(self, m, k, n, order=0):
+        """The launches of one matmul_q4_0_dequant_ordered."""
+        at = self.f.fake_launches()
+        self.m.check(self.lib.mri_matmul_q4_0_dequant_ordered(
+            X, (C.c_size_t * 2)(m, k), 2, W, n * k // 32 * 18, n, k, order, OUT, STREAM))
+        return self.launches(at)
+
+
+def check_q4_0_releases_no_workspace(h):
+    """A recorded graph of the Q8_0 GEMM's K split replays with the stream's
+    workspace: a later Q4_0 call on the stream, whose parts need more, leaves it."""
+    call = h.q8_0(200, 4096, 6000)
+    h.m.check(call())
+    held = h.live()
+    assert "k_gemm_q8_0" in h.launches()[-1][0]
+    launched = h.q4_0(256, 4096, 11008)
+    assert any("k_q4_0_gemm" in name for name, _ in launched)
+    assert held <= h.live()
+    for m in (512, 700):
+        h.q4_0(m, 11008, 4096)
+        assert held <= h.live()
+
+
+CHECKS = [n for n in dir() if n.startswith("check_")]
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake_hip") / "libfake_hip.so")
+    subprocess.run(["cc", "-O1", "-shared", "-fPIC", "-w", "-I/opt/rocm/include",
+                    os.path.join(HERE, "fake_hip.c"), "-o", so], check=True)
+    return so
+
+
+@pytest.mark.parametrize("check", CHECKS)
+def test_host(fake, check):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), fake, check],
+                       capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+if __name__ == "__main__":
+    globals()[sys.argv[2]](Host(sys.argv[1]))
