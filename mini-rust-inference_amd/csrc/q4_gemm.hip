@@ -47,16 +47,27 @@ constexpr int kXcds = 8;
 
 // Byte of 16-byte piece g of row r in a 64-byte-pitch LDS tile.
 __device__ inline int swz(int r, int g) { return r * 64 + ((g ^ ((r >> 1) & 3)) << 4); }
-template <int BM, int BN, int WM, int WN, int WK, int KB, int PD, bool GG>
+
+// The end of K part p of np, in blocks: even, so that every tile's stages end
+// there too (but for the last part's).
+__device__ inline int part_end(int nb, int p, int np) {
+    return min(2 * ((nb + 1) / 2 * (p + 1) / np), nb);
+}
+
+// The sum is of np K parts (plan_q4), added in part order: by np workgroups a
+// tile, which take one each and meet in a workspace, or (TURN) by one, which
+// takes them in turn, to the same bits.
+template <int BM, int BN, int WM, int WN, int WK, int KB, int PD, bool GG, bool TURN>
 __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q4_0_gemm(
     const float *__restrict__ x, int M, int K, const uint8_t *__restrict__ w, int N, int n_mt,
-    int n_total, int ks, float *__restrict__ out, float *__restrict__ part, int *__restrict__ cnt) {
+    int n_total, int np, float *__restrict__ out, float *__restrict__ part, int *__restrict__ cnt) {
     constexpr int NT = WM * WN * WK * 64;
     constexpr int RI = BM / 16 / WM, RJ = BN / 16 / WN;  // 16 x 16 sub-tiles of a wave
     constexpr int LA = BM * 8 * KB / NT;                 // float4 pieces a thread
     constexpr int UB = BN * 4 * KB, LB = (UB + NT - 1) / NT;  // 4-byte quant pieces
     constexpr int US = BN * KB, LS = (US + NT - 1) / NT;      // scales
     static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0 && BM * 8 * KB % NT == 0 && KB % WK == 0, "tile");
+    static_assert(WK > 1 || KB <= 2, "part_end");
     constexpr int SA = KB * 3 * BM * 64, SB = KB * BN * 64;
     constexpr int STAGE = SA + SB + US * 4;
     extern __shared__ uint4 s_q4[];
@@ -64,6 +75,7 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
 
     const int per_xcd = (int)(gridDim.x / kXcds);
     const int item = (int)(blockIdx.x % kXcds) * per_xcd + (int)(blockIdx.x / kXcds);
+    const int ks = TURN ? 1 : np;  // workgroups a tile
     if (item >= n_total * ks) return;
     const int tile = item / ks, kpart = item - tile * ks;
     const int mt = tile % n_mt, nt = tile / n_mt;
@@ -71,7 +83,8 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
     const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wk = wv / (WM * WN), wm = wv / WN % WM, wn = wv % WN;
     const int nb = K / 32, S = (nb + KB - 1) / KB;
-    const int s0 = (int)((long long)S * kpart / ks), s1 = (int)((long long)S * (kpart + 1) / ks);
+    const int s0 = kpart ? part_end(nb, kpart - 1, np) / KB : 0;
+    const int s1 = kpart + 1 < ks ? part_end(nb, kpart, np) / KB : S;
 
     // this thread's pieces of a stage: rows past M and channels past N read
     // the last one (their outputs are not stored); blocks past the end of K
@@ -217,6 +230,9 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
                         fs[i][j][e] = __builtin_fmaf(acc[i][j][e], d[j], fs[i][j][e]);
         }
     };
+    [[maybe_unused]] f4 tot[RI][RJ];  // TURN: the parts before this one
+    [[maybe_unused]] int p = 0, p_end = TURN ? part_end(nb, 0, np) / KB : 0;
+
     // Stage s lives in register set (s - s0) % PD until it is written to LDS.
     // The barrier waits for LDS only: the loads of the next PD stages stay
     // in flight across it.
@@ -234,7 +250,24 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
                 store(s + u + 1, regs[(u + 1) % PD]);
                 load(s + u + 1 + PD, regs[(u + 1) % PD]);
             }
+            if (TURN && s + u + 1 == p_end) {
+#pragma unroll
+                for (int i = 0; i < RI; ++i)
+#pragma unroll
+                    for (int j = 0; j < RJ; ++j) {
+                        tot[i][j] = p ? tot[i][j] + fs[i][j] : fs[i][j];
+                        fs[i][j] = f4{0, 0, 0, 0};
+                    }
+                ++p;
+                p_end = p + 1 < np ? part_end(nb, p, np) / KB : -1;
+            }
         }
+    }
+    if constexpr (TURN) {  // the last part
+#pragma unroll
+        for (int i = 0; i < RI; ++i)
+#pragma unroll
+            for (int j = 0; j < RJ; ++j) fs[i][j] = tot[i][j] + fs[i][j];
     }
 
     if constexpr (WK > 1) {
@@ -249,14 +282,14 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
                 red[(wk - 1) * BM * BN + i * 64] = fs[i / 4 / RJ][i / 4 % RJ][i % 4];
         }
         __syncthreads();
-        if (wk > 0) return;  // (never with ks > 1, whose barriers follow)
+        if (wk > 0) return;  // (never with np > 1, whose barriers follow)
 #pragma unroll
         for (int p = 0; p < WK - 1; ++p)
 #pragma unroll
             for (int i = 0; i < W; ++i)
                 fs[i / 4 / RJ][i / 4 % RJ][i % 4] += red[p * BM * BN + i * 64];
     }
-    if (WK == 1 && ks > 1) {
+    if (!TURN && WK == 1 && np > 1) {
         // K split: every part leaves its sums in its slot and counts itself
         // on the tile's counter; the last to arrive adds the parts in part
         // order.  Slots are written with device-scope stores, complete at
@@ -264,7 +297,7 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
         // device-scope loads.
         __shared__ int s_last;
         constexpr int W = RI * RJ * 4;
-        float *mine = part + ((size_t)tile * ks + kpart) * (BM * BN) + (size_t)wv * W * 64 + l;
+        float *mine = part + ((size_t)tile * np + kpart) * (BM * BN) + (size_t)wv * W * 64 + l;
 #pragma unroll
         for (int i = 0; i < RI; ++i)
 #pragma unroll
@@ -277,12 +310,12 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
         __syncthreads();
         if (t == 0)
             s_last = __hip_atomic_fetch_add(&cnt[tile], 1, __ATOMIC_RELAXED,
-                                            __HIP_MEMORY_SCOPE_AGENT) == ks - 1;
+                                            __HIP_MEMORY_SCOPE_AGENT) == np - 1;
         __syncthreads();
         if (!s_last) return;
         f4 tot[RI][RJ];
-        for (int p = 0; p < ks; ++p) {
-            const float *src = part + ((size_t)tile * ks + p) * (BM * BN) + (size_t)wv * W * 64 + l;
+        for (int p = 0; p < np; ++p) {
+            const float *src = part + ((size_t)tile * np + p) * (BM * BN) + (size_t)wv * W * 64 + l;
 #pragma unroll
             for (int i = 0; i < RI; ++i)
 #pragma unroll
@@ -318,11 +351,12 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
     }
 }
 
-template <int BM, int BN, int WM, int WN, int WK, int KB, int PD, bool GG>
-mri_status launch_cfg(const float *x, size_t m, size_t k, const uint8_t *w, size_t n, int ks,
+template <int BM, int BN, int WM, int WN, int WK, int KB, int PD, bool GG, bool TURN = false>
+mri_status launch_cfg(const float *x, size_t m, size_t k, const uint8_t *w, size_t n, int np,
                       float *out, void *ws, hipStream_t s) {
+    const int ks = TURN ? 1 : np;
     constexpr int lds = 2 * (KB * 3 * BM * 64 + KB * BN * 64 + BN * KB * 4);
-    auto kernel = &k_q4_0_gemm<BM, BN, WM, WN, WK, KB, PD, GG>;
+    auto kernel = &k_q4_0_gemm<BM, BN, WM, WN, WK, KB, PD, GG, TURN>;
     static DeviceOnce attr;
     MRI_HIP(attr.run([&](int) {
         return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
@@ -333,7 +367,7 @@ mri_status launch_cfg(const float *x, size_t m, size_t k, const uint8_t *w, size
     int *cnt = static_cast<int *>(ws);
     float *part = ws ? reinterpret_cast<float *>(cnt + kGemmWsCounters) : nullptr;
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(WM * WN * WK * 64), lds, s, x, (int)m,
-                       (int)k, w, (int)n, (int)n_mt, (int)total, ks, out, part, cnt);
+                       (int)k, w, (int)n, (int)n_mt, (int)total, np, out, part, cnt);
     MRI_LAUNCHED("k_q4_0_gemm");
     return MRI_OK;
 }
@@ -343,33 +377,34 @@ mri_status launch_cfg(const float *x, size_t m, size_t k, const uint8_t *w, size
 // back), in 0.01 us, measured at K = 4096 with 256-11008 channels.
 struct Tile {
     int bm, bn, block, part;
+    size_t count(size_t m, size_t n) const { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); }
 };
 constexpr Tile kTiles[] = {{64, 128, 55, 200}, {128, 128, 81, 350}, {128, 256, 117, 700}};
 constexpr int kMaxParts = 8, kMinPartBlocks = 8;
 
 // The tile and K split of least modelled time: passes of the CUs, times the
 // blocks of a part, plus the parts.  At 256 x 4096 x 11008 it takes 128 x 256
-// tiles in two parts (172 workgroups, one pass: 93 us; whole tiles 151), at
-// 512 x 4096 x 4096 128 x 128 in two (65 us; whole 104).
-void plan_q4(size_t m, size_t k, size_t n, bool may_split, int *tile, int *parts) {
+// tiles in two parts (172 workgroups, one pass), at 512 x 4096 x 4096
+// 128 x 128 in two.  The parts belong to the result (their sums are added in
+// part order), so they depend on the sizes alone; *whole is the better of the
+// first two tiles for one workgroup that takes all parts (the third one's
+// registers do not hold their totals too: 333 x 4096 x 12288 430 us, in
+// 128 x 128 tiles 215; split 143).
+void plan_q4(size_t m, size_t k, size_t n, int *tile, int *parts, int *whole) {
     const long long nb = (long long)(k / 32), cus = std::max(device_cus(), 1);
-    long long best = -1;
+    long long best = -1, best_whole = -1;
     for (int c = 0; c < 3; ++c) {
         const Tile &tl = kTiles[c];
-        const long long tiles =
-            (long long)((m + tl.bm - 1) / tl.bm) * (long long)((n + tl.bn - 1) / tl.bn);
-        for (int ks = 1; ks <= (may_split ? kMaxParts : 1); ++ks) {
+        const long long tiles = (long long)tl.count(m, n);
+        for (int ks = 1; ks <= kMaxParts; ++ks) {
             if (ks > 1 && (nb / ks < kMinPartBlocks || tiles > kGemmWsCounters ||
                            tiles * ks > 4 * cus))
                 break;
             const long long passes = (tiles * ks + cus - 1) / cus;
             const long long cost =
                 passes * ((nb + ks - 1) / ks) * tl.block + (ks > 1 ? ks * tl.part : 0);
-            if (best < 0 || cost < best) {
-                best = cost;
-                *tile = c;
-                *parts = ks;
-            }
+            if (best < 0 || cost < best) best = cost, *tile = c, *parts = ks;
+            if (ks == 1 && c < 2 && (best_whole < 0 || cost < best_whole)) best_whole = cost, *whole = c;
         }
     }
 }
@@ -394,26 +429,38 @@ mri_status launch_gemm(const float *x, size_t m, size_t k, const uint8_t *w, siz
             return launch_cfg<32, 32, 1, 2, 8, 8, 2, GG>(x, m, k, w, n, 1, out, nullptr, s);
         return launch_cfg<32, 64, 1, 4, 4, 4, 3, GG>(x, m, k, w, n, 1, out, nullptr, s);
     }
-    // A stream that is being captured gets no K split: no recorded graph holds
-    // the workspace, which may therefore grow at any later call.
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    bool may_split = hipStreamIsCapturing(s, &cap) == hipSuccess;
-    if (!may_split) (void)hipGetLastError();
-    may_split = may_split && cap == hipStreamCaptureStatusNone;
-    int tile = 0, parts = 1;
-    plan_q4(m, k, n, may_split, &tile, &parts);
-    void *ws = nullptr;
+    int tile = 0, parts = 1, whole = 0;
+    plan_q4(m, k, n, &tile, &parts, &whole);
     if (parts > 1) {
-        const Tile &tl = kTiles[tile];
-        const size_t tiles = ((m + tl.bm - 1) / tl.bm) * ((n + tl.bn - 1) / tl.bn);
-        const mri_status st = q4_ws_get(
-            s, kGemmWsCounters * sizeof(int) + tiles * parts * tl.bm * tl.bn * sizeof(float), &ws);
-        if (st) return st;
+        // A stream that is being captured gets no K split over workgroups: no
+        // recorded graph holds the workspace, which may therefore grow at any
+        // later call.  One workgroup a tile adds the same parts instead (split
+        // and not: 256 x 4096 x 11008 98 and 116 us, 64 x 4096 x 4096 20 and 74).
+        void *ws = nullptr;
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+            (void)hipGetLastError();
+            cap = hipStreamCaptureStatusActive;
+        }
+        if (cap == hipStreamCaptureStatusNone) {
+            const Tile &tl = kTiles[tile];
+            const mri_status st =
+                q4_ws_get(s, kGemmWsCounters * sizeof(int) +
+                                 tl.count(m, n) * parts * tl.bm * tl.bn * sizeof(float), &ws);
+            if (st) return st;
+        }
+        switch (ws ? tile : whole + 3) {
+        case 0: return launch_cfg<64, 128, 2, 4, 1, 2, 2, GG>(x, m, k, w, n, parts, out, ws, s);
+        case 1: return launch_cfg<128, 128, 4, 4, 1, 1, 2, GG>(x, m, k, w, n, parts, out, ws, s);
+        case 2: return launch_cfg<128, 256, 2, 8, 1, 1, 2, GG>(x, m, k, w, n, parts, out, ws, s);
+        case 3: return launch_cfg<64, 128, 2, 4, 1, 2, 2, GG, true>(x, m, k, w, n, parts, out, ws, s);
+        default: return launch_cfg<128, 128, 4, 4, 1, 1, 2, GG, true>(x, m, k, w, n, parts, out, ws, s);
+        }
     }
     switch (tile) {
-    case 0: return launch_cfg<64, 128, 2, 4, 1, 2, 2, GG>(x, m, k, w, n, parts, out, ws, s);
-    case 1: return launch_cfg<128, 128, 4, 4, 1, 1, 2, GG>(x, m, k, w, n, parts, out, ws, s);
-    default: return launch_cfg<128, 256, 2, 8, 1, 1, 2, GG>(x, m, k, w, n, parts, out, ws, s);
+    case 0: return launch_cfg<64, 128, 2, 4, 1, 2, 2, GG>(x, m, k, w, n, 1, out, nullptr, s);
+    case 1: return launch_cfg<128, 128, 4, 4, 1, 1, 2, GG>(x, m, k, w, n, 1, out, nullptr, s);
+    default: return launch_cfg<128, 256, 2, 8, 1, 1, 2, GG>(x, m, k, w, n, 1, out, nullptr, s);
     }
 }
 

@@ -154,3 +154,28 @@ def test_recorded_graph_outlives_a_larger_call():
             want4 = host(out4)
             check(want4, host(x4), raw, n4, k4)
         assert_bits_equal(host(out4), want4, "Q4_0 beside the graph")
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (128, 512, 4096), (256, 11008, 4096), (512, 4096, 4096), (65, 300, 2080),
+    (33, 129, 1056), (200, 515, 11008), (64, 4100, 544)])
+def test_captured_call_has_the_eager_bits(m, n, k):
+    """A captured call, which has no workspace, adds the K parts of the eager
+    one in the same order (the last sizes: stages of two blocks, odd block
+    counts), on rows and channels that fill no tile."""
+    t = torch()
+    rng = np.random.default_rng(m + n + k)
+    raw = synth_q4_0(rng, n, k)
+    xd, w = dev((rng.standard_normal((m, k)) * np.exp(rng.standard_normal(k))).astype(F32)), dev(raw)
+    out, cap = empty((m, n), t.float32), t.full((m + 1, n), 7.0, device="cuda")
+    mri().matmul_q4_0_dequant(xd, w, n, k, out)
+    t.cuda.synchronize()
+    g = t.cuda.CUDAGraph()
+    with t.cuda.graph(g, stream=t.cuda.Stream()):
+        mri().matmul_q4_0_dequant(xd, w, n, k, cap[:m])
+    for _ in range(2):
+        cap[:m].fill_(float("nan"))
+        g.replay()
+        got = host(cap)
+        assert_bits_equal(got[:m], host(out), "captured")
+        assert np.all(got[m] == 7.0)
