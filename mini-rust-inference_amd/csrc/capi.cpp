@@ -148,8 +148,44 @@ mri_status gemm_ws_get(hipStream_t stream, size_t bytes, void **ptr) {
     return zeroed_ws_get(g_ws, stream, bytes, ptr);
 }
 
+// While it lives, this thread may take and give back memory beside captures of
+// other streams, which in the default mode such calls would break.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 mri_status q4_ws_get(hipStream_t stream, size_t bytes, void **ptr) {
-    return zeroed_ws_get(g_q4ws, stream, bytes, ptr);
+    int dev = 0;
+    MRI_HIP(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    Scratch &sc = g_q4ws[{dev, stream}];
+    *ptr = nullptr;
+    if (sc.bytes < bytes) {
+        const RelaxedCapture relaxed;
+        const size_t want = round_up(bytes, 1u << 20);
+        void *p = nullptr;
+        if (hipMalloc(&p, want) != hipSuccess) {
+            (void)hipGetLastError();
+            return MRI_OK;
+        }
+        // on the stream itself: the default stream would wait for captures
+        const mri_status st = launch_zero(p, kGemmWsCounters, stream);
+        if (st) {
+            (void)hipFree(p);
+            return st;
+        }
+        void *old = sc.ptr;
+        sc.ptr = p;
+        sc.bytes = want;
+        if (old) {
+            MRI_HIP(hipStreamSynchronize(stream));
+            MRI_HIP(hipFree(old));
+        }
+    }
+    *ptr = sc.ptr;
+    return MRI_OK;
 }
 
 mri_status argmax_ws_get(hipStream_t stream, void **ptr, size_t bytes) {

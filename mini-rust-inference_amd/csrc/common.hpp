@@ -372,10 +372,12 @@ bool gemm_rows_ok(size_t m, const QMatrixDev &w, const void *act);
 // (re)allocated.
 mri_status gemm_ws_get(hipStream_t stream, size_t bytes, void **ptr);
 // The Q4_0 GEMM's, for calls that are not being captured: [kGemmWsCounters
-// tile counters][f32 partial tiles].
+// tile counters][f32 partial tiles].  *ptr is null where the memory cannot be
+// had.
 mri_status q4_ws_get(hipStream_t stream, size_t bytes, void **ptr);
 
 // q4_0.hip
+mri_status launch_zero(void *p, size_t words, hipStream_t s);  // 4-byte words
 mri_status launch_q4_0_dequant(const float *x, size_t m, size_t k, const uint8_t *w,
                                size_t n_out, bool ggml_order, float *out, hipStream_t s);
 

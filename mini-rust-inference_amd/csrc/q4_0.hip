@@ -189,9 +189,10 @@ __global__ __launch_bounds__(NW * 64) void k_q4_0_gemv(const float *__restrict__
     }
 }
 
-__global__ __launch_bounds__(kThreads) void k_q4_0_empty(size_t n, float *__restrict__ out) {
-    const size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x;
-    if (i < n) out[i] = 0.0f;
+__global__ __launch_bounds__(kThreads) void k_zero(size_t n, unsigned *__restrict__ p) {
+    for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < n;
+         i += (size_t)gridDim.x * kThreads)
+        p[i] = 0;
 }
 
 template <int R, bool GG>
@@ -343,13 +344,7 @@ mri_status launch_gemv_rows(const float *x, size_t m, size_t k, const uint8_t *w
 template <bool GG>
 mri_status launch_q4(const float *x, size_t m, size_t k, const uint8_t *w, size_t n_out,
                      float *out, hipStream_t s) {
-    if (k == 0) {
-        const size_t n = m * n_out;
-        hipLaunchKernelGGL(k_q4_0_empty, dim3((unsigned)((n + kThreads - 1) / kThreads)),
-                           dim3(kThreads), 0, s, n, out);
-        MRI_LAUNCHED("k_q4_0_empty");
-        return MRI_OK;
-    }
+    if (k == 0) return launch_zero(out, m * n_out, s);
     const size_t cus = (size_t)std::max(device_cus(), 1), tiles = (n_out + 15) / 16;
     const bool few = 2 * tiles <= 3 * cus;  // 16-channel workgroups fit about one a CU
     // the staged form: 16-byte aligned rows (K % 256 == 0) and operands
@@ -378,6 +373,14 @@ mri_status launch_q4(const float *x, size_t m, size_t k, const uint8_t *w, size_
 }
 
 }  // namespace
+
+mri_status launch_zero(void *p, size_t words, hipStream_t s) {
+    const size_t grid = std::min<size_t>((words + kThreads - 1) / kThreads, 65536);
+    hipLaunchKernelGGL(k_zero, dim3((unsigned)grid), dim3(kThreads), 0, s, words,
+                       static_cast<unsigned *>(p));
+    MRI_LAUNCHED("k_zero");
+    return MRI_OK;
+}
 
 mri_status launch_q4_0_dequant(const float *x, size_t m, size_t k, const uint8_t *w,
                                size_t n_out, bool ggml_order, float *out, hipStream_t s) {

@@ -21,8 +21,20 @@ static dim3 cfg_grid, cfg_block;
 static size_t cfg_lds;
 static hipStream_t cfg_stream;
 
-/* what the tests set */
-int fake_refuse_malloc, fake_capturing;
+/* what the tests set: refuse memory; the call's stream is being captured;
+ * another stream is, in global mode, which a call that takes, gives back or
+ * waits for something in that mode breaks */
+int fake_refuse_malloc, fake_capturing, fake_other_capture;
+int fake_broken_captures;
+static hipStreamCaptureMode mode = hipStreamCaptureModeGlobal;
+static int unsafe(void) {
+    if (!fake_other_capture || mode == hipStreamCaptureModeRelaxed) return 0;
+    return ++fake_broken_captures;
+}
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *m) {
+    hipStreamCaptureMode was = mode;
+    return mode = *m, *m = was, hipSuccess;
+}
 
 int fake_allocs(void) { return n_allocs; }
 int fake_live(int i) { return allocs[i].live; }
@@ -35,6 +47,7 @@ const char *fake_launch(int i, unsigned v[6]) {
 }
 
 hipError_t hipMalloc(void **p, size_t n) {
+    if (unsafe()) return hipErrorStreamCaptureUnsupported;
     if (fake_refuse_malloc || n_allocs == MAX) return hipErrorOutOfMemory;
     allocs[n_allocs].p = next, allocs[n_allocs].n = n, allocs[n_allocs].live = 1;
     ++n_allocs;
@@ -43,6 +56,7 @@ hipError_t hipMalloc(void **p, size_t n) {
     return hipSuccess;
 }
 hipError_t hipFree(void *p) {
+    if (unsafe()) return hipErrorStreamCaptureUnsupported;
     for (int i = 0; i < n_allocs; ++i)
         if (allocs[i].p == (uintptr_t)p && allocs[i].live) {
             allocs[i].live = 0;
@@ -61,7 +75,9 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *p, int d) {
     return hipSuccess;
 }
 hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t s) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) {
+    return unsafe() ? hipErrorStreamCaptureUnsupported : hipSuccess;
+}
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *c) {
     return *c = fake_capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone,
            hipSuccess;
@@ -78,7 +94,9 @@ hipError_t hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t
                             hipMemcpyKind k, hipStream_t t) {
     return hipSuccess;
 }
-hipError_t hipMemset(void *p, int v, size_t n) { return hipSuccess; }
+hipError_t hipMemset(void *p, int v, size_t n) {
+    return unsafe() ? hipErrorStreamCaptureUnsupported : hipSuccess;
+}
 hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t s) { return hipSuccess; }
 
 /* the compiler's registration and launch entries */

@@ -179,3 +179,27 @@ def test_captured_call_has_the_eager_bits(m, n, k):
         got = host(cap)
         assert_bits_equal(got[:m], host(out), "captured")
         assert np.all(got[m] == 7.0)
+
+
+def test_eager_call_beside_a_capture():
+    """An eager call whose workspace must grow while another stream of the
+    thread is being captured: the bits are the same, and the capture ends well."""
+    t = torch()
+    rng = np.random.default_rng(10)
+    n, k = 11008, 4096
+    raw = synth_q4_0(rng, n, k)
+    w, out, want = dev(raw), empty((256, n), t.float32), empty((256, n), t.float32)
+    x = dev(rng.standard_normal((256, k)).astype(F32))
+    mri().matmul_q4_0_dequant(x, w, n, k, want)
+    y = t.ones(8, device="cuda")
+    t.cuda.synchronize()
+    a, b = t.cuda.Stream(), t.cuda.Stream()
+    g = t.cuda.CUDAGraph()
+    with t.cuda.graph(g, stream=a):
+        y.add_(1)
+        with t.cuda.stream(b):
+            mri().matmul_q4_0_dequant(x, w, n, k, out)
+    t.cuda.synchronize()
+    assert_bits_equal(host(out), host(want), "beside a capture")
+    g.replay()
+    assert host(y).tolist() == [2.0] * 8

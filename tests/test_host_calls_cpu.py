@@ -67,6 +67,34 @@ def check_q4_0_releases_no_workspace(h):
         assert held <= h.live()
 
 
+def check_q4_0_without_memory(h):
+    """A Q4_0 call whose K parts' memory is refused runs without the split, and
+    a workspace that is too small for it stays."""
+    h.q4_0(64, 1024, 1024)
+    held = h.live()
+    h.set("fake_refuse_malloc", 1)
+    (whole, _), = h.q4_0(256, 4096, 11008)
+    assert "k_q4_0_gemm" in whole and held == h.live()
+    small, = h.q4_0(64, 1024, 1024)      # what is there is used
+    h.set("fake_refuse_malloc", 0)
+    split = h.q4_0(256, 4096, 11008)[-1][0]
+    assert split != whole and len(h.live()) == 1
+    assert h.q4_0(64, 1024, 1024) == [small]
+    h.set("fake_capturing", 1)           # a captured call: the unsplit form too
+    assert h.q4_0(256, 4096, 11008)[0][0] == whole
+
+
+def check_q4_0_beside_a_capture(h):
+    """An eager Q4_0 call that takes or grows its workspace while another
+    stream is being captured leaves that capture whole."""
+    h.set("fake_other_capture", 1)
+    h.q4_0(64, 1024, 1024)
+    split = h.q4_0(256, 4096, 11008)[-1]
+    assert C.c_int.in_dll(h.f, "fake_broken_captures").value == 0
+    h.set("fake_other_capture", 0)
+    assert h.q4_0(256, 4096, 11008) == [split]
+
+
 CHECKS = [n for n in dir() if n.startswith("check_")]
 
 
