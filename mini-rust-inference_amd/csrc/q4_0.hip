@@ -69,17 +69,18 @@ size_t q4_gemv_lds(int m, int nw, size_t k) {
 template <int M, int NW, bool GG>
 __global__ __launch_bounds__(NW * 64) void k_q4_0_gemv(const float *__restrict__ x, int K,
                                                        const uint8_t *__restrict__ w, int N,
-                                                       float *__restrict__ out) {
+                                                       int tile0, float *__restrict__ out) {
     constexpr int NT = NW * 64;
     extern __shared__ u4 s_x[];
     const int t = threadIdx.x, l = t & 63;
     const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const int nb = K / 32, Q = (nb + 3) / 4;
     const int r = l & 15, g = l >> 4;
+    const int n0 = 16 * (tile0 + (int)blockIdx.x);
     const int plane = Q * 16;  // 16-byte pieces
     const int zero = M * 3 * plane;
     // channels past N read the last one (not stored)
-    const uint8_t *row = w + (size_t)min(16 * (int)blockIdx.x + r, N - 1) * nb * kQ4Bytes;
+    const uint8_t *row = w + (size_t)min(n0 + r, N - 1) * nb * kQ4Bytes;
 
     // The 18 bytes of this lane's block of a lap (blocks past the end: the
     // last one, counted as zero): the 4-byte aligned words around its quants
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(NW * 64) void k_q4_0_gemv(const float *__restrict__
     }
     __syncthreads();
     if (t < 16 * M) {
-        const int m = t >> 4, n = 16 * blockIdx.x + (t & 15);
+        const int m = t >> 4, n = n0 + (t & 15);
         float s = red[m * NW * 16 + (t & 15)];
 #pragma unroll
         for (int v = 1; v < NW; ++v) s += red[(m * NW + v) * 16 + (t & 15)];
@@ -310,9 +311,14 @@ mri_status launch_lds(const float *x, size_t k, const uint8_t *w, size_t n_out,
         return hipFuncSetAttribute(reinterpret_cast<const void *>(&k_q4_0_lds<R, GG>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
     }));
-    hipLaunchKernelGGL((k_q4_0_lds<R, GG>), dim3((unsigned)((n_out + R - 1) / R)),
-                       dim3(kThreads), q4_lds_bytes(R, k), s, x, (int)k, w, (int)n_out, out);
-    MRI_LAUNCHED("k_q4_0_lds");
+    const size_t step = R * q4_max_grid(kThreads);
+    for (size_t n = 0; n < n_out; n += step) {
+        const size_t c = std::min(n_out - n, step);
+        hipLaunchKernelGGL((k_q4_0_lds<R, GG>), dim3((unsigned)((c + R - 1) / R)), dim3(kThreads),
+                           q4_lds_bytes(R, k), s, x, (int)k, w + n * (k / 32) * kQ4Bytes, (int)c,
+                           out + n);
+        MRI_LAUNCHED("k_q4_0_lds");
+    }
     return MRI_OK;
 }
 
@@ -324,9 +330,13 @@ mri_status launch_gemv(const float *x, size_t k, const uint8_t *w, size_t n_out,
         return hipFuncSetAttribute(reinterpret_cast<const void *>(&k_q4_0_gemv<M, NW, GG>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
     }));
-    hipLaunchKernelGGL((k_q4_0_gemv<M, NW, GG>), dim3((unsigned)((n_out + 15) / 16)),
-                       dim3(NW * 64), q4_gemv_lds(M, NW, k), s, x, (int)k, w, (int)n_out, out);
-    MRI_LAUNCHED("k_q4_0_gemv");
+    const size_t tiles = (n_out + 15) / 16, step = q4_max_grid(NW * 64);
+    for (size_t t = 0; t < tiles; t += step) {
+        hipLaunchKernelGGL((k_q4_0_gemv<M, NW, GG>), dim3((unsigned)std::min(tiles - t, step)),
+                           dim3(NW * 64), q4_gemv_lds(M, NW, k), s, x, (int)k, w, (int)n_out,
+                           (int)t, out);
+        MRI_LAUNCHED("k_q4_0_gemv");
+    }
     return MRI_OK;
 }
 

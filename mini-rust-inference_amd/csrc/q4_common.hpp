@@ -33,4 +33,8 @@ __device__ inline void q4_quants(unsigned w, float (&l)[4], float (&h)[4]) {
     l[2] = q4_quant<0>(v), h[2] = q4_quant<4>(v), l[3] = q4_quant<8>(v), h[3] = q4_quant<12>(v);
 }
 
+// Workgroups of one launch, a multiple of 8: HIP takes fewer than 2^32 threads
+// in a grid dimension, which 2^27 channels exceed.  More take more launches.
+inline size_t q4_max_grid(size_t threads) { return 0xFFFFFFFFull / threads / 8 * 8; }
+
 }  // namespace mri

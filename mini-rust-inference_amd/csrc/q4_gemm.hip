@@ -60,7 +60,7 @@ __device__ inline int part_end(int nb, int p, int np) {
 template <int BM, int BN, int WM, int WN, int WK, int KB, int PD, bool GG, bool TURN>
 __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q4_0_gemm(
     const float *__restrict__ x, int M, int K, const uint8_t *__restrict__ w, int N, int n_mt,
-    int n_total, int np, float *__restrict__ out, float *__restrict__ part, int *__restrict__ cnt) {
+    int n_total, int np, int item0, float *__restrict__ out, float *__restrict__ part, int *__restrict__ cnt) {
     constexpr int NT = WM * WN * WK * 64;
     constexpr int RI = BM / 16 / WM, RJ = BN / 16 / WN;  // 16 x 16 sub-tiles of a wave
     constexpr int LA = BM * 8 * KB / NT;                 // float4 pieces a thread
@@ -74,7 +74,7 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
     char *lds = reinterpret_cast<char *>(s_q4);
 
     const int per_xcd = (int)(gridDim.x / kXcds);
-    const int item = (int)(blockIdx.x % kXcds) * per_xcd + (int)(blockIdx.x / kXcds);
+    const int item = item0 + (int)(blockIdx.x % kXcds) * per_xcd + (int)(blockIdx.x / kXcds);
     const int ks = TURN ? 1 : np;  // workgroups a tile
     if (item >= n_total * ks) return;
     const int tile = item / ks, kpart = item - tile * ks;
@@ -366,9 +366,13 @@ mri_status launch_cfg(const float *x, size_t m, size_t k, const uint8_t *w, size
     const size_t grid = (total * ks + kXcds - 1) / kXcds * kXcds;
     int *cnt = static_cast<int *>(ws);
     float *part = ws ? reinterpret_cast<float *>(cnt + kGemmWsCounters) : nullptr;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(WM * WN * WK * 64), lds, s, x, (int)m,
-                       (int)k, w, (int)n, (int)n_mt, (int)total, np, out, part, cnt);
-    MRI_LAUNCHED("k_q4_0_gemm");
+    constexpr int threads = WM * WN * WK * 64;
+    for (size_t i = 0; i < grid; i += q4_max_grid(threads)) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(grid - i, q4_max_grid(threads))),
+                           dim3(threads), lds, s, x, (int)m, (int)k, w, (int)n, (int)n_mt,
+                           (int)total, np, (int)i, out, part, cnt);
+        MRI_LAUNCHED("k_q4_0_gemm");
+    }
     return MRI_OK;
 }
 

@@ -203,3 +203,25 @@ def test_eager_call_beside_a_capture():
     assert_bits_equal(host(out), host(want), "beside a capture")
     g.replay()
     assert host(y).tolist() == [2.0] * 8
+
+
+@pytest.mark.parametrize("m,n", [(1, 2**27 + 40), (3, 2**28 + 40)])
+def test_channels_past_one_launch(m, n):
+    """More channels than one launch has threads for: the first, the last and
+    those around the second launch's first are what a call on them alone gives."""
+    t = torch()
+    k, g = 32, t.Generator(device="cuda")
+    g.manual_seed(m)
+    raw = t.randint(0, 2**31 - 1, (n * 18 // 4,), dtype=t.int32, device="cuda", generator=g)
+    raw = raw.view(t.uint8).view(n, 18)
+    raw[:, 1] = 0x1C    # scales of 2^-8 to 2^-7
+    x = t.randn(m, k, device="cuda", generator=g)
+    out = t.empty(m, n, device="cuda")
+    mri().matmul_q4_0_dequant(x, raw.view(-1), n, k, out)
+    per = 16 * ((2**32 - 1) // 512 // 8 * 8) if m == 1 else 64 * ((2**32 - 1) // 1024 // 8 * 8)
+    part = t.empty(m, 136, device="cuda")
+    for a in (0, n // 2, min(per - 64, n - 136), n - 136):
+        mri().matmul_q4_0_dequant(x, raw[a:a + 136].reshape(-1), 136, k, part)
+        check(host(part), host(x), host(raw[a:a + 136]).ravel(), 136, k)
+        got = host(out[:, a:a + 136].contiguous())
+        assert np.linalg.norm(got - host(part)) <= 1e-6 * np.linalg.norm(host(part)), a

@@ -95,6 +95,23 @@ def check_q4_0_beside_a_capture(h):
     assert h.q4_0(256, 4096, 11008) == [split]
 
 
+def check_q4_0_grids(h):
+    """HIP launches fewer than 2^32 threads in a grid dimension: more channels
+    or rows than that take several launches, whose workgroups cover them all."""
+    for m, k, n, channels, rows in (
+            (1, 32, 2**27 + 40, 16, 1), (2, 32, 2**28, 16, 2),       # a workgroup's outputs
+            (1, 256, 2**27 + 40, 8, 1), (1, 256, 2**30, 8, 1),
+            (3, 32, 2**28 + 40, 64, 16), (17, 32, 2**28 + 40, 64, 32),
+            (1, 32, 2**31 - 1024, 64, 16), (2**29, 32, 1, 128, 128), (2**30, 0, 3, None, None)):
+        launched = h.q4_0(m, k, n)
+        for name, v in launched:
+            assert v[0] * v[3] < 2**32, (m, k, n, name, v)
+        if channels:
+            need = -(-m // rows) * -(-n // channels)
+            got = sum(v[0] for _, v in launched)
+            assert need <= got < need + 8, (m, k, n, launched)
+
+
 CHECKS = [n for n in dir() if n.startswith("check_")]
 
 
