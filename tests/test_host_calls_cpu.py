@@ -44,6 +44,16 @@ class Host:
         return lambda: self.lib.mri_matmul_q8_0_direct(X, (C.c_size_t * 2)(m, k), 2, h, OUT,
                                                        None, None, STREAM)
 
+    def w4a8(self, m, k, n):
+        """The launches of one matmul_q4_0_w4a8."""
+        h = C.c_void_p()
+        self.m.check(self.lib.mri_q4_0_matrix_from_raw_device(W, n * k // 32 * 18, n, k, 0,
+                                                              STREAM, C.byref(h)))
+        at = self.f.fake_launches()
+        self.m.check(self.lib.mri_matmul_q4_0_w4a8(X, (C.c_size_t * 2)(m, k), 2, h, OUT, None,
+                                                   None, STREAM))
+        return self.launches(at)
+
     def q4_0(self, m, k, n, order=0):
         """The launches of one matmul_q4_0_dequant_ordered."""
         at = self.f.fake_launches()
@@ -110,6 +120,15 @@ def check_q4_0_grids(h):
             need = -(-m // rows) * -(-n // channels)
             got = sum(v[0] for _, v in launched)
             assert need <= got < need + 8, (m, k, n, launched)
+
+
+def check_block_grids(h):
+    """As above, for the quantized rows of W4A8 past the LDS-tiled kernel."""
+    for m, n in ((2**21, 2**13), (2**21 + 5, 2**13 + 1), (2**17, 2**17)):
+        launched = [(name, v) for name, v in h.w4a8(m, 32, n) if "k_skinny" in name]
+        for name, v in launched:
+            assert v[0] * v[3] < 2**32, (m, n, name, v)
+        assert sum(v[0] * v[3] // 64 for _, v in launched) >= -(-m // 16) * -(-n // 16)
 
 
 CHECKS = [n for n in dir() if n.startswith("check_")]
