@@ -19,7 +19,8 @@
 // the activations of block 4 lap + g and is zero elsewhere; the four MFMAs
 // add up to register p of lane (r, g) = plane p's sum of its own block, which
 // it adds (smallest first) and scales by the d that it loaded.  The planes
-// are split once per workgroup into LDS.  Bound: the unpacking (2.6 VALU
+// are split once per workgroup into LDS; bits below 2^-133, which they do not
+// hold, are added in f32 where there are any (as in q4_gemm.hip).  Bound: the unpacking (2.6 VALU
 // operations a weight) and its loads, 72-byte pieces of 16 rows.  It took
 // 1 x 4128 x 11008 from 23.4 to 10.4 us (the earlier two-lanes-a-block f32
 // kernel), 2 x 4128 x 8000 from 33.1 to 9.2 and 4 x 992 x 512 from 12.9 to
@@ -59,11 +60,14 @@ constexpr int kThreads = 256;
 constexpr int kMaxLds = 160 * 1024;
 
 // LDS of k_q4_0_gemv: [M][3 planes][4 Q blocks][64 bytes] and a 16-byte zero
-// line; the reduction's M * NW * 16 floats fit in it (NW <= 16, Q >= 1: 768 M
-// bytes and more).
+// line, whose place the M * NW * 16 floats of the reduction take, then a flag
+// a wave.
+__host__ __device__ inline size_t q4_gemv_flags(int m, int nw, size_t q) {
+    const size_t planes = (size_t)m * 3 * q * 256 + 16, red = (size_t)m * nw * 64;
+    return planes > red ? planes : red;
+}
 size_t q4_gemv_lds(int m, int nw, size_t k) {
-    const size_t q = (k / 32 + 3) / 4;
-    return std::max((size_t)m * 3 * q * 256 + 16, (size_t)m * nw * 64);
+    return q4_gemv_flags(m, nw, (k / 32 + 3) / 4) + 4 * nw;
 }
 
 template <int M, int NW, bool GG>
@@ -104,6 +108,8 @@ __global__ __launch_bounds__(NW * 64) void k_q4_0_gemv(const float *__restrict__
         a = *reinterpret_cast<const f4 *>(p + (GG ? 4 * j : 8 * j));
         b = *reinterpret_cast<const f4 *>(p + (GG ? 16 + 4 * j : 8 * j + 4));
     };
+    // bits that the planes do not hold leave a trace in the low half of `lost`
+    unsigned lost = 0;
     auto put = [&](int m, int u, f4 a, f4 b) __attribute__((always_inline)) {
         if (u >= 4 * nb) a = b = f4{0, 0, 0, 0};
         f4 lo = GG ? a : f4{a[0], a[2], b[0], b[2]};
@@ -114,12 +120,19 @@ __global__ __launch_bounds__(NW * 64) void k_q4_0_gemv(const float *__restrict__
                                               q4_top16(hi[0], hi[1]), q4_top16(hi[2], hi[3])};
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
+                if (p == 2) lost |= __float_as_uint(lo[e]) | __float_as_uint(hi[e]);
                 lo[e] -= q4_cut(lo[e]);
                 hi[e] -= q4_cut(hi[e]);
             }
         }
     };
     const int units = 16 * Q;
+    int *flag = reinterpret_cast<int *>(s_x) + q4_gemv_flags(M, NW, Q) / 4;
+    float acc[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m) acc[m] = 0.0f;
+    const bool on = (r >> 2) == g && (r & 3) < 3;
+    const int st = on ? 1 : 0;
     f4 xa[M], xb[M];
 #pragma unroll
     for (int m = 0; m < M; ++m) get(m, min(t, units - 1), xa[m], xb[m]);
@@ -139,11 +152,6 @@ __global__ __launch_bounds__(NW * 64) void k_q4_0_gemv(const float *__restrict__
     // LDS only: the weight loads stay in flight
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
 
-    float acc[M];
-#pragma unroll
-    for (int m = 0; m < M; ++m) acc[m] = 0.0f;
-    const bool on = (r >> 2) == g && (r & 3) < 3;
-    const int st = on ? 1 : 0;
     for (int lap = wv; lap < Q; lap += NW) {
         const int blk = 4 * lap + g;
         const float ds = blk < nb ? f16_bits_to_f32(d) : 0.0f;
@@ -172,22 +180,50 @@ __global__ __launch_bounds__(NW * 64) void k_q4_0_gemv(const float *__restrict__
         }
     }
     // the four lane groups' blocks, then the waves' laps in wave order
-    __syncthreads();
-    float *red = reinterpret_cast<float *>(s_x);
+    auto finish = [&]() __attribute__((always_inline)) {
+        float *red = reinterpret_cast<float *>(s_x);
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
-        acc[m] += __shfl_xor(acc[m], 16);
-        acc[m] += __shfl_xor(acc[m], 32);
-        if (l < 16) red[(m * NW + wv) * 16 + l] = acc[m];
+        for (int m = 0; m < M; ++m) {
+            float s = acc[m] + __shfl_xor(acc[m], 16);
+            s += __shfl_xor(s, 32);
+            if (l < 16) red[(m * NW + wv) * 16 + l] = s;
+        }
+        __syncthreads();
+        if (t < 16 * M) {
+            const int m = t >> 4, n = n0 + (t & 15);
+            float s = red[m * NW * 16 + (t & 15)];
+#pragma unroll
+            for (int v = 1; v < NW; ++v) s += red[(m * NW + v) * 16 + (t & 15)];
+            if (n < N) out[(size_t)m * N + n] = s;
+        }
+    };
+    const bool mine = __any(lost & 0xFFFFu);
+    if (l == 0) flag[wv] = mine;
+    __syncthreads();
+    const int any = flag[min(l, NW - 1)];
+    finish();
+    if (!__any(any)) return;
+    // rare: the lost bits' products (q4_rest) in f32, lane (r, g)'s of channel
+    // r and every (4 NW)-th block
+#pragma unroll 1
+    for (int b = t >> 4; b < nb; b += NT / 16) {
+        const uint8_t *p = row + (size_t)b * kQ4Bytes;
+        const float ds =
+            q4_rest_scale(f16_bits_to_f32(*reinterpret_cast<const uint16_t *>(p)));
+        float c[M] = {};
+#pragma unroll 1
+        for (int e = 0; e < 32; ++e) {
+            const int nib = GG ? p[2 + (e & 15)] >> (e >> 4) * 4 : p[2 + (e >> 1)] >> (e & 1) * 4;
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+                c[m] = __builtin_fmaf(q4_rest(x[(size_t)m * K + 32 * b + e]),
+                                      (float)((nib & 15) - 8), c[m]);
+        }
+#pragma unroll
+        for (int m = 0; m < M; ++m) acc[m] = __builtin_fmaf(c[m], ds, acc[m]);
     }
     __syncthreads();
-    if (t < 16 * M) {
-        const int m = t >> 4, n = n0 + (t & 15);
-        float s = red[m * NW * 16 + (t & 15)];
-#pragma unroll
-        for (int v = 1; v < NW; ++v) s += red[(m * NW + v) * 16 + (t & 15)];
-        if (n < N) out[(size_t)m * N + n] = s;
-    }
+    finish();
 }
 
 __global__ __launch_bounds__(kThreads) void k_zero(size_t n, unsigned *__restrict__ p) {

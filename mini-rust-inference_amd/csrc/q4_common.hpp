@@ -4,17 +4,29 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+
 namespace mri {
 
 // An f32 value is exactly the sum of three bf16 values: its leading 8
 // significand bits, the next 8 and the last 8, each cut off (not rounded)
-// from what the ones before leave.  cut() is the part a bf16 holds; top16()
-// stores the parts of two values as a bf16 pair (a low, b high).
+// from what the ones before leave, down to 2^-133, a bf16's last bit.  cut() is
+// the part a bf16 holds; top16() stores the parts of two values as a bf16 pair
+// (a low, b high).  rest() is 2^64 times what the three leave of a value (its
+// bits below 2^-133), rest_scale() the block scale that undoes the factor.
 __device__ inline float q4_cut(float v) {
     return __uint_as_float(__float_as_uint(v) & 0xFFFF0000u);
 }
 __device__ inline unsigned q4_top16(float a, float b) {
     return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+__device__ inline float q4_rest(float v) {
+    v -= q4_cut(v);
+    v -= q4_cut(v);
+    return (v - q4_cut(v)) * 0x1p64f;
+}
+__device__ inline float q4_rest_scale(float d) {
+    return fabsf(d) < INFINITY ? d * 0x1p-64f : 0.0f;
 }
 
 // The quant (nibble - 8) of the nibble at bit P <= 12 of w, exactly: the

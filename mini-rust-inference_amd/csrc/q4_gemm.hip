@@ -9,7 +9,10 @@
 // so every product of the three planes with the quants is exact, and
 // v_mfma_f32_16x16x32_bf16 adds them in f32: three MFMAs a block (smallest
 // plane first), then one FMA with the block's scale.  Infinities and NaNs
-// give NaN, as the regrouped sums of the other Q4_0 kernels do.
+// give NaN, as the regrouped sums of the other Q4_0 kernels do.  Bits below
+// 2^-133, which bf16 does not hold, are seen while splitting (values below
+// 2^-109 can have them); a workgroup that met any goes over its K again with
+// those bits alone, 2^64 times them, and its scales 2^-64 times.
 //
 // A workgroup computes BM rows x BN channels.  A stage is KB blocks of K:
 // its f32 activations and quant bytes are loaded into registers one stage
@@ -29,6 +32,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "q4_common.hpp"
@@ -44,6 +48,11 @@ struct __attribute__((packed, aligned(2))) U32a2 {
 };
 
 constexpr int kXcds = 8;
+
+// A barrier that waits for the wave's LDS accesses only.
+__device__ inline void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+}
 
 // Byte of 16-byte piece g of row r in a 64-byte-pitch LDS tile.
 __device__ inline int swz(int r, int g) { return r * 64 + ((g ^ ((r >> 1) & 3)) << 4); }
@@ -82,9 +91,11 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
     const int t = threadIdx.x, l = t & 63;
     const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wk = wv / (WM * WN), wm = wv / WN % WM, wn = wv % WN;
-    const int nb = K / 32, S = (nb + KB - 1) / KB;
-    const int s0 = kpart ? part_end(nb, kpart - 1, np) / KB : 0;
-    const int s1 = kpart + 1 < ks ? part_end(nb, kpart, np) / KB : S;
+    const int nb = K / 32;
+    // the stages of K part q are [first(q), first(q + 1))
+    auto first = [&](int q) __attribute__((always_inline)) {
+        return q == 0 ? 0 : q == np ? (nb + KB - 1) / KB : part_end(nb, q - 1, np) / KB;
+    };
 
     // this thread's pieces of a stage: rows past M and channels past N read
     // the last one (their outputs are not stored); blocks past the end of K
@@ -123,7 +134,7 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
         unsigned b[LB];
         unsigned s[LS];
     } regs[PD];
-    auto load = [&](int s, Regs &r) __attribute__((always_inline)) {
+    auto load = [&](int s, Regs &r, int s1) __attribute__((always_inline)) {
         const int b0 = min(s, s1 - 1) * KB;
 #pragma unroll
         for (int i = 0; i < LA; ++i)
@@ -137,7 +148,11 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
             r.s[i] = *reinterpret_cast<const uint16_t *>(s_src[i] +
                                                         kQ4Bytes * min(b0 + s_kb[i], nb - 1));
     };
-    auto store = [&](int s, const Regs &r) __attribute__((always_inline)) {
+    // REST: of the bits that the planes do not hold (q4_rest); otherwise their
+    // presence is left in the low half of `lost`.
+    unsigned lost = 0;
+    auto store = [&](int s, const Regs &r, int s0, auto rest) __attribute__((always_inline)) {
+        constexpr bool REST = decltype(rest)::value;
         char *buf = lds + ((s - s0) & 1) * STAGE;
         const int b0 = s * KB;
 #pragma unroll
@@ -147,8 +162,10 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
             float md[4], lo[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
+                if constexpr (REST) v[e] = q4_rest(v[e]);
                 md[e] = v[e] - q4_cut(v[e]);
                 lo[e] = md[e] - q4_cut(md[e]);
+                if constexpr (!REST) lost |= __float_as_uint(lo[e]);
             }
             char *p = buf + a_dst[i];
             *reinterpret_cast<uint2 *>(p) = uint2{q4_top16(v[0], v[1]), q4_top16(v[2], v[3])};
@@ -179,7 +196,8 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
 #pragma unroll
         for (int i = 0; i < LS; ++i) {
             if (US % NT && t + NT * i >= US) continue;
-            const float d = f16_bits_to_f32(r.s[i]);
+            float d = f16_bits_to_f32(r.s[i]);
+            if constexpr (REST) d = q4_rest_scale(d);
             *reinterpret_cast<float *>(buf + s_dst[i]) = KB > 1 && b0 + s_kb[i] >= nb ? 0.0f : d;
         }
     };
@@ -194,7 +212,7 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
     const int b_off = SA + swz(wn * RJ * 16 + fr, fg);
     const int d_off = SA + SB + (wn * RJ * 16 + fr) * 4;
 
-    auto product = [&](int s) __attribute__((always_inline)) {
+    auto product = [&](int s, int s0) __attribute__((always_inline)) {
         const char *buf = lds + ((s - s0) & 1) * STAGE;
 #pragma unroll
         for (int k = 0; k < KB / WK; ++k) {
@@ -230,44 +248,80 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
                         fs[i][j][e] = __builtin_fmaf(acc[i][j][e], d[j], fs[i][j][e]);
         }
     };
-    [[maybe_unused]] f4 tot[RI][RJ];  // TURN: the parts before this one
-    [[maybe_unused]] int p = 0, p_end = TURN ? part_end(nb, 0, np) / KB : 0;
-
-    // Stage s lives in register set (s - s0) % PD until it is written to LDS.
-    // The barrier waits for LDS only: the loads of the next PD stages stay
-    // in flight across it.
-#pragma unroll
-    for (int u = 0; u < PD; ++u) load(s0 + u, regs[u]);
-    store(s0, regs[0]);
-    load(s0 + PD, regs[0]);
-    for (int s = s0; s < s1; s += PD) {
-#pragma unroll
-        for (int u = 0; u < PD; ++u) {
-            if (s + u >= s1) break;
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
-            product(s + u);
-            if (s + u + 1 < s1) {
-                store(s + u + 1, regs[(u + 1) % PD]);
-                load(s + u + 1 + PD, regs[(u + 1) % PD]);
-            }
-            if (TURN && s + u + 1 == p_end) {
-#pragma unroll
-                for (int i = 0; i < RI; ++i)
-#pragma unroll
-                    for (int j = 0; j < RJ; ++j) {
-                        tot[i][j] = p ? tot[i][j] + fs[i][j] : fs[i][j];
-                        fs[i][j] = f4{0, 0, 0, 0};
-                    }
-                ++p;
-                p_end = p + 1 < np ? part_end(nb, p, np) / KB : -1;
-            }
-        }
-    }
-    if constexpr (TURN) {  // the last part
+    // K split: this workgroup's slot of the workspace (see below)
+    auto put = [&]() __attribute__((always_inline)) {
+        constexpr int W = RI * RJ * 4;
+        float *mine = part + ((size_t)tile * np + kpart) * (BM * BN) + (size_t)wv * W * 64 + l;
 #pragma unroll
         for (int i = 0; i < RI; ++i)
 #pragma unroll
-            for (int j = 0; j < RJ; ++j) fs[i][j] = tot[i][j] + fs[i][j];
+            for (int j = 0; j < RJ; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    __hip_atomic_store(mine + ((i * RJ + j) * 4 + e) * 64, fs[i][j][e],
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    };
+    const bool split = !TURN && WK == 1 && np > 1;
+    __shared__ int s_lost[NT / 64];
+    [[maybe_unused]] f4 tot[RI][RJ];  // TURN: the parts so far
+    // Stage s lives in register set (s - s0) % PD until it is written to LDS.
+    // The barrier waits for LDS only: the loads of the next PD stages stay
+    // in flight across it.
+    for (int p = kpart;;) {
+        const int s0 = first(p), s1 = first(p + 1);
+#pragma unroll
+        for (int u = 0; u < PD; ++u) load(s0 + u, regs[u], s1);
+        store(s0, regs[0], s0, std::false_type{});
+        load(s0 + PD, regs[0], s1);
+        for (int s = s0; s < s1; s += PD) {
+#pragma unroll
+            for (int u = 0; u < PD; ++u) {
+                if (s + u >= s1) break;
+                lds_barrier();
+                product(s + u, s0);
+                if (s + u + 1 < s1) {
+                    store(s + u + 1, regs[(u + 1) % PD], s0, std::false_type{});
+                    load(s + u + 1 + PD, regs[(u + 1) % PD], s1);
+                }
+            }
+        }
+        // (the next write of a flag is a barrier or more away)
+        const bool mine = __any(lost & 0xFFFFu);
+        if (l == 0) s_lost[wv] = mine;
+        if (split) put();
+        lds_barrier();
+        if (__any(s_lost[min(l, NT / 64 - 1)])) {
+            // rare, so not pipelined: a second pipelined loop, or one loop for
+            // both with a branch in store(), cost every call 3-12 %; this 0-1
+            for (int s = s0; s < s1; ++s) {
+                load(s, regs[0], s1);
+                store(s, regs[0], s, std::true_type{});
+                lds_barrier();
+                product(s, s);
+                lds_barrier();
+            }
+            lost = 0;
+            if (split) {
+                put();
+                lds_barrier();
+            }
+        }
+        if constexpr (!TURN) break;
+#pragma unroll
+        for (int i = 0; i < RI; ++i)
+#pragma unroll
+            for (int j = 0; j < RJ; ++j) {
+                tot[i][j] = p ? tot[i][j] + fs[i][j] : fs[i][j];
+                fs[i][j] = f4{0, 0, 0, 0};
+            }
+        if (++p == np) break;
+    }
+    if constexpr (TURN) {
+#pragma unroll
+        for (int i = 0; i < RI; ++i)
+#pragma unroll
+            for (int j = 0; j < RJ; ++j) fs[i][j] = tot[i][j];
     }
 
     if constexpr (WK > 1) {
@@ -289,7 +343,7 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
             for (int i = 0; i < W; ++i)
                 fs[i / 4 / RJ][i / 4 % RJ][i % 4] += red[p * BM * BN + i * 64];
     }
-    if (!TURN && WK == 1 && np > 1) {
+    if (split) {
         // K split: every part leaves its sums in its slot and counts itself
         // on the tile's counter; the last to arrive adds the parts in part
         // order.  Slots are written with device-scope stores, complete at
@@ -297,17 +351,6 @@ __global__ __launch_bounds__(WM *WN *WK * 64, WM * WN * WK > 8 ? 4 : 2) void k_q
         // device-scope loads.
         __shared__ int s_last;
         constexpr int W = RI * RJ * 4;
-        float *mine = part + ((size_t)tile * np + kpart) * (BM * BN) + (size_t)wv * W * 64 + l;
-#pragma unroll
-        for (int i = 0; i < RI; ++i)
-#pragma unroll
-            for (int j = 0; j < RJ; ++j)
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    __hip_atomic_store(mine + ((i * RJ + j) * 4 + e) * 64, fs[i][j][e],
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-        __syncthreads();
         if (t == 0)
             s_last = __hip_atomic_fetch_add(&cnt[tile], 1, __ATOMIC_RELAXED,
                                             __HIP_MEMORY_SCOPE_AGENT) == np - 1;

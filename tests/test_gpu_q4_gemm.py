@@ -225,3 +225,48 @@ def test_channels_past_one_launch(m, n):
         check(host(part), host(x), host(raw[a:a + 136]).ravel(), 136, k)
         got = host(out[:, a:a + 136].contiguous())
         assert np.linalg.norm(got - host(part)) <= 1e-6 * np.linalg.norm(host(part)), a
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 40, 1056), (2, 33, 96), (4, 25, 4128), (3, 31, 8192),        # per block, 8 and 16 waves
+    (5, 17, 288), (7, 6200, 544), (17, 33, 288), (18, 8300, 320),    # 16 and 32 rows
+    (64, 127, 1056), (130, 1000, 4096), (256, 11008, 4096)])         # 64- and 128-row tiles, parts
+@pytest.mark.parametrize("ggml", [False, True])
+def test_activations_below_the_planes(m, n, k, ggml):
+    """Activations down to 2^-149, whose last bits bf16 does not hold, in every
+    row or in one block of one row, eager and captured.  Scales of 1 to 2 keep
+    the results' own f32 steps (2^-150 a rounding) below the bound: sums of
+    terms of 2^-126 and more, at most 344 roundings."""
+    t = torch()
+    rng = np.random.default_rng(m * 7 + n + k)
+    raw = synth_q4_0(rng, n, k).reshape(-1, 18)
+    raw[:, 1] = 0x3C
+    raw = raw.ravel()
+    order = mri().Q4_ORDER_GGML if ggml else mri().Q4_ORDER_INTERLEAVED
+    w = dev(CF.q4_0_interleaved_to_ggml(raw) if ggml else raw)
+    out, cap = empty((m, n), t.float32), empty((m, n), t.float32)
+    one = rng.standard_normal((m, k))
+    for e in (-118, -131):
+        x = np.ldexp(one, e).astype(F32)
+        part = rng.standard_normal((m, k)).astype(F32)
+        part[m // 2, :-32] = 0
+        part[m // 2, -32:] = x[m // 2, -32:]
+        for v in (x, part):
+            xd = dev(v)
+            mri().matmul_q4_0_dequant_ordered(xd, w, n, k, order, out)
+            check(host(out), v, raw, n, k)
+            g = t.cuda.CUDAGraph()
+            with t.cuda.graph(g, stream=t.cuda.Stream()):
+                mri().matmul_q4_0_dequant_ordered(xd, w, n, k, order, cap)
+            for _ in range(2):
+                g.replay()
+                assert_bits_equal(host(cap), host(out), "captured")
+    x = np.ldexp(one[0], -131).astype(F32)   # and beside a scale that is not finite
+    raw = raw.copy().reshape(n, -1, 18)
+    raw[0, 0, :2] = 0, 0x7C
+    raw[0, 0, 2:] = 0xFF
+    x[:32] = np.abs(x[:32])
+    xd = dev(np.broadcast_to(x, (m, k)).copy())
+    w = dev(CF.q4_0_interleaved_to_ggml(raw.ravel()) if ggml else raw.ravel())
+    mri().matmul_q4_0_dequant_ordered(xd, w, n, k, order, out)
+    assert np.all(host(out)[:, 0] == np.inf)
