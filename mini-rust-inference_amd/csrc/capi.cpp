@@ -673,8 +673,8 @@ mri_status mri_quantize_symmetric(const float *x, size_t len, int8_t *q, float *
     void *base = nullptr;
     st = scratch_get(s, 1024 * sizeof(float), &base);
     if (st) return st;
-    return launch_quantize_tensor(x, 1, len, len, false, nullptr, q, scale,
-                                  static_cast<float *>(base), s);
+    return launch_quantize_tensor(x, 1, len, len, nullptr, q, scale, static_cast<float *>(base),
+                                  s);
 }
 
 mri_status mri_quantize_symmetric_rows(const float *x, size_t m, size_t k, int8_t *q,
@@ -830,7 +830,7 @@ mri_status mri_matmul_int8_from_f32(const float *input, const size_t *dims, size
         }
         return launch_gemm_int8(act, m, scale, 0, 0.0f, d, out, acc_out, ws, s);
     }
-    st = launch_quantize_tensor(input, m, k, d.kp, false, act, act_q_out, scale, partials, s);
+    st = launch_quantize_tensor(input, m, k, d.kp, act, act_q_out, scale, partials, s);
     if (st) return st;
     if (m * d.n_out == 0) return MRI_OK;
     return run_int8(act, m, scale, 0, 0.0f, d, out, acc_out, s);

@@ -201,10 +201,9 @@ mri_status scratch_get(hipStream_t stream, size_t bytes, void **ptr);
 
 // ---- kernel launchers (defined in the .hip files) -------------------------
 // quantize.hip
-mri_status launch_quantize_tensor(const float *x, size_t m, size_t k,
-                                  size_t ld_out, bool q8_perm_layout,
-                                  int8_t *q_pad, int8_t *q_plain,
-                                  float *scale, float *partials,
+// up to 65535 rows
+mri_status launch_quantize_tensor(const float *x, size_t m, size_t k, size_t ld_out,
+                                  int8_t *q_pad, int8_t *q_plain, float *scale, float *partials,
                                   hipStream_t s);
 // mg > 0: q_pad in the row-group layout (act_groups) instead of rows.
 mri_status launch_quantize_rows(const float *x, size_t m, size_t k,

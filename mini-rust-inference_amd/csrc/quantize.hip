@@ -9,6 +9,7 @@
 // The library is compiled with -ffp-contract=off and correctly rounded
 // f32 division, so each operation rounds exactly once, as in Rust.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -77,14 +78,15 @@ __device__ inline float absmax4(float m, const float4 &v) {
 __device__ inline float swiglu_elem(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 
 // quantize_symmetric of [m][k] with one scale: blockIdx.y a row, the threads
-// of blockIdx.x its elements, four at a time (VEC: float4 rows and 4-byte
-// aligned int8 rows) or one.  q_pad: [m][ld] (ld >= k, zero padded;
-// chunk-permuted when perm) or null; q_plain: [m*k] row-major or null.
+// of blockIdx.x its elements, W at a time (VEC: as a float4, of float4 rows and
+// 4-byte aligned int8 rows; else element by element, with one store of four
+// where the output row is aligned).  q_pad: [m][ld] (ld >= k, zero padded) or
+// null; q_plain: [m*k] row-major or null.
 // n_partials > 0: the maximum comes from k_absmax_partial; 0: every workgroup
 // reads the whole tensor (n elements) for it, which saves that launch.
-template <bool VEC>
+template <bool VEC, int W>
 __global__ __launch_bounds__(kTensorThreads) void k_quantize_tensor(
-    const float *__restrict__ x, size_t n, size_t k, size_t ld, int perm,
+    const float *__restrict__ x, size_t n, size_t k, size_t ld,
     const float *__restrict__ partials, int n_partials,
     int8_t *__restrict__ q_pad, int8_t *__restrict__ q_plain,
     float *__restrict__ scale_out) {
@@ -93,19 +95,28 @@ __global__ __launch_bounds__(kTensorThreads) void k_quantize_tensor(
     float mx = 0.0f;
     if (n_partials > 0) {
         for (int i = (int)t; i < n_partials; i += kTensorThreads) mx = fmaxf(mx, partials[i]);
-    } else if (VEC) {
-        const float4 *x4 = reinterpret_cast<const float4 *>(x);
-        constexpr int D = 8;  // loads in flight a thread
-        for (size_t i = t; i < n / 4; i += D * kTensorThreads) {
-            float4 v[D];
-#pragma unroll
-            for (int u = 0; u < D; ++u)  // past the end: the last one again
-                v[u] = x4[min(i + u * kTensorThreads, n / 4 - 1)];
-#pragma unroll
-            for (int u = 0; u < D; ++u) mx = absmax4(mx, v[u]);
-        }
     } else {
-        for (size_t i = t; i < n; i += kTensorThreads) mx = fmaxf(mx, fabsf(x[i]));
+        // float4s from the first aligned element on, the others (threads 0-2 and
+        // 4-6) one by one
+        const size_t head =
+            VEC ? 0 : min((size_t)(-(reinterpret_cast<uintptr_t>(x) >> 2) & 3), n);
+        const size_t n4 = (n - head) / 4, tail = n - head - 4 * n4;
+        if (!VEC && (t < head || t - 4 < tail)) mx = fabsf(x[t < head ? t : n + 3 - t]);
+        const float4 *x4 = reinterpret_cast<const float4 *>(x + head);
+        auto scan = [&](auto d) __attribute__((always_inline)) {
+            constexpr int D = decltype(d)::value;  // loads in flight a thread
+            for (size_t i = t; i < n4; i += D * kTensorThreads) {
+                float4 v[D];
+#pragma unroll
+                for (int u = 0; u < D; ++u)  // past the end: the last one again
+                    v[u] = x4[min(i + u * kTensorThreads, n4 - 1)];
+#pragma unroll
+                for (int u = 0; u < D; ++u) mx = absmax4(mx, v[u]);
+            }
+        };
+        if (n4 <= kTensorThreads) scan(std::integral_constant<int, 1>{});
+        else if (n4 <= 2 * kTensorThreads) scan(std::integral_constant<int, 2>{});
+        else scan(std::integral_constant<int, 8>{});
     }
     mx = block_max(mx, red);
     const float scale = scale_of(mx);
@@ -113,28 +124,31 @@ __global__ __launch_bounds__(kTensorThreads) void k_quantize_tensor(
     if (blockIdx.x == 0 && blockIdx.y == 0 && t == 0 && scale_out) *scale_out = scale;
     const size_t r = blockIdx.y;
     const float *row = x + r * k;
-    constexpr size_t W = VEC ? 4 : 1;
+    int8_t *pad = q_pad ? q_pad + r * ld : nullptr, *plain = q_plain ? q_plain + r * k : nullptr;
     const size_t step = (size_t)gridDim.x * kTensorThreads * W;
     for (size_t kk = (blockIdx.x * (size_t)kTensorThreads + t) * W; kk < ld; kk += step) {
+        float v[W] = {};
         if constexpr (VEC) {
-            int packed = 0;
-            if (kk < k) {
-                const float4 v = *reinterpret_cast<const float4 *>(row + kk);
-                packed = ((int)round_clamp_i8(v.x * inv) & 255) |
-                         (((int)round_clamp_i8(v.y * inv) & 255) << 8) |
-                         (((int)round_clamp_i8(v.z * inv) & 255) << 16) |
-                         ((int)round_clamp_i8(v.w * inv) << 24);
-                if (q_plain) *reinterpret_cast<int *>(q_plain + r * k + kk) = packed;
-            }
-            if (q_pad) *reinterpret_cast<int *>(q_pad + act_pos(r, kk, ld, perm, 0)) = packed;
+            if (kk < k) *reinterpret_cast<float4 *>(v) = *reinterpret_cast<const float4 *>(row + kk);
         } else {
-            int8_t q = 0;
-            if (kk < k) {
-                q = round_clamp_i8(row[kk] * inv);
-                if (q_plain) q_plain[r * k + kk] = q;
-            }
-            if (q_pad) q_pad[act_pos(r, kk, ld, perm, 0)] = q;
+#pragma unroll
+            for (int e = 0; e < W; ++e)
+                if (kk + e < k) v[e] = row[kk + e];
         }
+        int packed = 0;
+#pragma unroll
+        for (int e = 0; e < W; ++e) packed |= ((int)round_clamp_i8(v[e] * inv) & 255) << (8 * e);
+        auto put = [&](int8_t *q, size_t end) __attribute__((always_inline)) {
+            if (VEC || (W == 4 && kk + 4 <= end && (reinterpret_cast<uintptr_t>(q + kk) & 3) == 0)) {
+                if (kk < end) *reinterpret_cast<int *>(q + kk) = packed;
+            } else {
+#pragma unroll
+                for (int e = 0; e < W; ++e)
+                    if (kk + e < end) q[kk + e] = (int8_t)(packed >> (8 * e));
+            }
+        };
+        if (pad) put(pad, ld);
+        if (plain) put(plain, k);
     }
 }
 
@@ -406,10 +420,8 @@ size_t quantize_partials_count(size_t n) {
     return g;
 }
 
-mri_status launch_quantize_tensor(const float *x, size_t m, size_t k,
-                                  size_t ld_out, bool q8_perm_layout,
-                                  int8_t *q_pad, int8_t *q_plain,
-                                  float *scale, float *partials,
+mri_status launch_quantize_tensor(const float *x, size_t m, size_t k, size_t ld_out,
+                                  int8_t *q_pad, int8_t *q_plain, float *scale, float *partials,
                                   hipStream_t s) {
     const size_t n = m * k;
     size_t ld = q_pad ? ld_out : k;
@@ -417,7 +429,6 @@ mri_status launch_quantize_tensor(const float *x, size_t m, size_t k,
         m = 1;
         k = ld = 0;
     }
-    if (m > 65535) return set_error(MRI_ERR_UNSUPPORTED, "quantize: more than 65535 rows");
     int g = 0;
     if (n > kOnePassElems) {
         g = (int)quantize_partials_count(n);
@@ -427,15 +438,25 @@ mri_status launch_quantize_tensor(const float *x, size_t m, size_t k,
     const bool vec = k % 4 == 0 && ld % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
                      (reinterpret_cast<uintptr_t>(q_pad) & 3) == 0 &&
                      (reinterpret_cast<uintptr_t>(q_plain) & 3) == 0;
-    const size_t per = (size_t)kTensorThreads * (vec ? 4 : 1);
-    const size_t gx = std::min<size_t>(std::max<size_t>((ld + per - 1) / per, 1), 4096);
+    // Rows that are not float4s: an element a thread up to two workgroups a CU
+    // and where they stride over the rows anyway; between, four, fewer
+    // workgroups finding the maximum (us a quantization, one and four: 10001
+    // elements 4.3 and 5.0, 100001 6.0 and 6.7, 1048577 9.7 and 7.1, 2^24 - 1
+    // 40.1 and 41.3).
+    constexpr size_t most = 4096;
+    const size_t ones = (ld + kTensorThreads - 1) / kTensorThreads;
+    const bool four =
+        vec || (m * ones > 2 * (size_t)std::max(device_cus(), 1) && ones <= most);
+    const size_t per = (size_t)kTensorThreads * (four ? 4 : 1);
+    const size_t gx = std::min(std::max<size_t>((ld + per - 1) / per, 1), most);
     const dim3 grid((unsigned)gx, (unsigned)m);
-    if (vec)
-        hipLaunchKernelGGL(k_quantize_tensor<true>, grid, dim3(kTensorThreads), 0, s, x, n, k, ld,
-                           q8_perm_layout ? 1 : 0, partials, g, q_pad, q_plain, scale);
-    else
-        hipLaunchKernelGGL(k_quantize_tensor<false>, grid, dim3(kTensorThreads), 0, s, x, n, k,
-                           ld, q8_perm_layout ? 1 : 0, partials, g, q_pad, q_plain, scale);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kTensorThreads), 0, s, x, n, k, ld, partials, g,
+                           q_pad, q_plain, scale);
+    };
+    if (vec) go(k_quantize_tensor<true, 4>);
+    else if (four) go(k_quantize_tensor<false, 4>);
+    else go(k_quantize_tensor<false, 1>);
     MRI_LAUNCHED("k_quantize_tensor");
     return MRI_OK;
 }

@@ -38,6 +38,7 @@ def test_rows_bit_exact(m, n, k):
     assert np.all(got[m] == 7.0)
     assert np.array_equal(host(acc), acc0)
     assert np.array_equal(host(qx).ravel(), np.asarray(q0).ravel())
+    assert_bits_equal(host(sx), np.asarray([s0], F32), "scale")
     out2 = empty((m, n), t.float32)  # without the optional outputs
     M.matmul_int8_from_f32(dev(x), w, out2)
     assert_bits_equal(host(out2), ref, "from f32, plain")
@@ -53,3 +54,26 @@ def test_no_rows_leave_a_scale():
     M.matmul_int8_from_f32(empty((0, 64), t.float32), w, empty((0, 16), t.float32),
                            act_scale_out=sx)
     assert host(sx)[0] == 1.0
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 7, 4093, 9001, 65535, 65536, 65537, 600001, 1048577])
+def test_tensor_of_any_length_and_alignment(n):
+    """The maximum and the rounding of one tensor at every float alignment of
+    the input and byte alignment of the output, with the largest value at either
+    end; element by element, four at a time, one pass and two launches."""
+    import mri_qmatmul as M
+    t = torch()
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal(n).astype(F32)
+    buf, sx = t.zeros(n + 4, device="cuda"), empty(1, t.float32)
+    q = t.full((n + 8,), 77, dtype=t.int8, device="cuda")
+    for off in range(4):
+        x[(off % 2) * (n - 1)] = -7.5 - off
+        q0, s0 = O.quantize_symmetric(x)
+        buf[off:off + n] = dev(x)
+        q.fill_(77)
+        M.quantize_symmetric(buf[off:off + n], q[off + 1:off + 1 + n], sx)
+        got = host(q)
+        assert_bits_equal(host(sx), np.asarray([s0], F32), "scale")
+        assert np.array_equal(got[off + 1:off + 1 + n], q0)
+        assert np.all(got[:off + 1] == 77) and np.all(got[off + 1 + n:] == 77)

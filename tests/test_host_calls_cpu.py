@@ -131,6 +131,17 @@ def check_block_grids(h):
         assert sum(v[0] * v[3] // 64 for _, v in launched) >= -(-m // 16) * -(-n // 16)
 
 
+def check_quantize_grids(h):
+    """A long tensor that is not whole aligned float4s takes the workgroups of
+    one that is: each of them finds the maximum again."""
+    def grid(x, n):
+        at = h.f.fake_launches()
+        h.m.check(h.lib.mri_quantize_symmetric(x, n, OUT, W, STREAM))
+        return h.launches(at)[-1][1]
+    for n in (1048576, 2**22 - 4):
+        assert grid(X, n + 1)[0] <= grid(X, n)[0] + 1 and grid(X + 4, n) == grid(X, n)
+
+
 CHECKS = [n for n in dir() if n.startswith("check_")]
 
 
