@@ -877,22 +877,6 @@ static mri_status matmul_blocks(const char *name, const float *input, const size
     if (m * k && !input) return set_error(MRI_ERR_INVALID_ARGUMENT, "input is null");
     if (m * d.n_out && !out) return set_error(MRI_ERR_INVALID_ARGUMENT, "out is null");
     if (m == 0) return MRI_OK;
-    // Rows are independent.  In slices where one launch of the skinny kernel
-    // (the one for so many outputs), 64 threads a 16 x 16 outputs, would pass
-    // HIP's 2^32 threads.
-    if (d.n_out && m > 16 && m >= ((size_t)1 << 34) / d.n_out &&
-        !(fixed && round_up(m * d.kp, 256) + m * sizeof(float) > MRI_NOALLOC_SCRATCH_BYTES)) {
-        const size_t step = std::max<size_t>(((size_t)1 << 33) / d.n_out / 16 * 16, 16);
-        for (size_t i = 0; i < m; i += step) {
-            const size_t part[2] = {std::min(step, m - i), k};
-            const mri_status st = matmul_blocks(
-                name, input + i * k, part, 2, d, out + i * d.n_out,
-                block_dots_out ? block_dots_out + i * d.n_out * d.n_blocks : nullptr,
-                act_scales_out ? act_scales_out + i : nullptr, stream, fixed, true);
-            if (st) return st;
-        }
-        return MRI_OK;
-    }
     int dev;
     mri_status st = current_device(&dev);
     if (st) return st;

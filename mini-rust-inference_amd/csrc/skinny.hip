@@ -1,6 +1,6 @@
-// skinny.hip — decode-shaped (INT8: 5..63 rows; Q8_0 and W4A8: 5..32 rows per
-// launch, and prefill sizes below the LDS-tiled GEMM's) quantized matmul on
-// CDNA4 MFMA.
+// skinny.hip — quantized matmul on CDNA4 MFMA for INT8 at 5..63 rows and, for
+// Q8_0 and W4A8, from 5 rows up to the sizes of the LDS-tiled GEMM (and at
+// every row count where the reference's block order is asked for).
 //
 // The weight stream dominates (M*K activation bytes vs N*K weight bytes), so
 // both kernels stream the 1 KiB weight chunks of 16-row tiles
@@ -151,9 +151,9 @@ __global__ __launch_bounds__(S * kWave) void k_skinny_int8(
 }
 
 // ---------------------------------------------------------------------------
-// Q8_0: AG groups of 16 activation rows a wave.  One wave per tile
-// of 16 output channels sweeps all of K in laps of one scale group (4
-// chunks = 8 blocks) and keeps RL laps of loads in flight: per chunk one
+// Q8_0: AG groups of 16 activation rows and NT tiles of 16 output channels a
+// wave, which sweeps all of K in laps of one scale group (4
+// chunks = 8 blocks) and keeps RL laps of loads in flight: per chunk and tile one
 // 16-byte load of the weight chunk and, per activation group, one 16-byte
 // load of the rows' matching activation bytes (chunk-permuted, so its two
 // halves are the A operands of the chunk's two blocks).  Per block and
@@ -162,47 +162,51 @@ __global__ __launch_bounds__(S * kWave) void k_skinny_int8(
 // running sums in block order (q8_direct.rs:269-282), so the f32 result is
 // bit-identical.  The sweep has no global memory instruction other than the
 // ring's loads and no data-dependent branch, so every wait leaves the
-// younger loads in flight.  Rows m >= M read row 0's activations; their
-// results are never stored.
+// younger loads in flight.  Rows m >= M read row 0's activations, or in row
+// groups what lies in the last group; their results are never stored.
 //
 // W4 (Q4_0 weights of the W4A8 path): a lap's quants are two 16-byte pieces
 // per lane; the 8-byte B operand of block h of chunk c is the u32 word
 // 2(c % 2) + h of piece c / 2 with each nibble moved to the high half of its
 // byte (16 * quant as int8), and the MFMA result is divided by 16 exactly.
 // ---------------------------------------------------------------------------
-template <int AG, int TPW, int RL, int CS, bool DEBUG, bool W4>
-__global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
+template <int AG, int NT, int RL, int CS, bool DEBUG, bool W4>
+__global__ __launch_bounds__(kWave) void k_skinny_q8_0(
     const int8_t *__restrict__ act, int M, int kp, const float *__restrict__ sa_rows,
     const v4i *__restrict__ laps, int N, int n_tiles, int G, int nb, float *__restrict__ out,
     int32_t *__restrict__ block_dots, int ns, int mg) {
-    // wave -> (tile, set of AG activation groups); the ns waves of a tile are
-    // adjacent, so they share a workgroup (or neighbouring ones) and the weight
-    // chunks they all stream are fetched from HBM once.
-    // With several workgroups per tile the grid (a multiple of 8) is
-    // taken XCD-major: workgroups are dispatched to the 8 XCDs round-robin,
-    // and consecutive indices of one XCD share its L2.
-    int blk = blockIdx.x;
-    if (ns > TPW) blk = (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8);
-    const int wv = blk * TPW + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int T = wv / ns;
-    const int a0 = (wv - T * ns) * AG;  // first activation group of the wave
-    if (T >= n_tiles) return;  // whole waves only; the kernel has no barrier
-    const int l = threadIdx.x & 63;
+    // wave -> (NT adjacent tiles, set of AG activation groups); the ns waves of
+    // the tiles are adjacent, so that the weight chunks they all stream are
+    // fetched from HBM once.  With several waves per tile the grid (a multiple
+    // of 8) is taken XCD-major: workgroups are dispatched to the 8 XCDs
+    // round-robin, and consecutive indices of one XCD share its L2.
+    int wv = blockIdx.x;
+    if (ns > 1) wv = (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8);
+    const int T0 = wv / ns * NT;
+    const int a0 = wv % ns * AG;  // first activation group of the wave
+    if (T0 >= n_tiles) return;  // whole waves only; the kernel has no barrier
+    const int l = threadIdx.x;
     const int r = l & 15, g = l >> 4;
-    // the tile's lap blocks: quant piece c of lap q at v4i offset
-    // q * LB + c * 64 (+ lane), the lap's scales at q * LB + SO (+ row)
+    // a tile's lap blocks: quant piece c of lap q at v4i offset
+    // q * LB + c * 64 (+ lane), the lap's scales at q * LB + SO (+ row); tiles
+    // past the end read the last one and store nothing
     constexpr size_t LB = (W4 ? kQ4LapBytes : kQ8LapBytes) / 16;
     constexpr int SO = W4 ? 128 : 256;
     constexpr int NP = W4 ? 2 : 4;  // quant pieces per lap and lane
     // (addresses as a wave-uniform base and a 32-bit lane offset, so that no
     // vector instruction goes into them: a wave that is alone on its SIMD is
     // bound by those it issues)
-    const char *wp = reinterpret_cast<const char *>(laps + (size_t)T * G * LB);
+    const char *wp[NT];
+    int n[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        wp[t] = reinterpret_cast<const char *>(laps + (size_t)min(T0 + t, n_tiles - 1) * G * LB);
+        n[t] = T0 + t < n_tiles ? (T0 + t) * 16 + r : N;
+    }
     const unsigned wl = 16 * l, sl = 16 * (SO + r);
     auto at = [](const char *base, unsigned lane) __attribute__((always_inline)) {
         return reinterpret_cast<const v4i *>(base + (size_t)lane);
     };
-    const int n = T * 16 + r;
     // the activations: this lane's 16 bytes of chunk p of its rows at
     // act + p * cs + al[a], in rows (past M: row 0) or in mg row groups.  CS
     // states the stride for one group or rows, where it is known: a lap's four
@@ -210,7 +214,7 @@ __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
     unsigned al[AG];
     const size_t cs = CS ? CS : mg ? (size_t)mg * 1024 : 64;
     const char *ap = reinterpret_cast<const char *>(act);
-    float sa[AG][4], fs[AG][4];
+    float sa[AG][4], fs[AG][NT][4];
 #pragma unroll
     for (int a = 0; a < AG; ++a) {
         const int m = 16 * (a0 + a) + r;
@@ -219,23 +223,28 @@ __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             sa[a][i] = sa_rows[min(16 * (a0 + a) + 4 * g + i, M - 1)];
-            fs[a][i] = 0.0f;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) fs[a][t][i] = 0.0f;
         }
     }
-    v4i wr[RL][4];
+    v4i wr[RL][NT][4];
     v4i xr[RL][4][AG];
-    v4i sr[RL];
+    v4i sr[RL][NT];
 #pragma unroll
     for (int u = 0; u < RL; ++u) {
         const int q = min(u, G - 1);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            if (c < NP)
-                wr[u][c] = __builtin_nontemporal_load(at(wp + ((size_t)q * LB + c * 64) * 16, wl));
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+                if (c < NP)
+                    wr[u][t][c] =
+                        __builtin_nontemporal_load(at(wp[t] + ((size_t)q * LB + c * 64) * 16, wl));
 #pragma unroll
             for (int a = 0; a < AG; ++a) xr[u][c][a] = *at(ap + (size_t)(4 * q + c) * cs, al[a]);
         }
-        sr[u] = *at(wp + (size_t)q * LB * 16, sl);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) sr[u][t] = *at(wp[t] + (size_t)q * LB * 16, sl);
     }
     const v4i zero = {0, 0, 0, 0};
     // Without W4 each block's MFMA starts from the bits of 1.5 * 2^23, so an
@@ -250,26 +259,29 @@ __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
         constexpr int U = decltype(slot)::value;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            v4i d[2][AG];
+            v4i d[2][AG][NT];
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                long bv;
-                if constexpr (W4) {
-                    const v4i pc = wr[U][c >> 1];
-                    const int wd = (c & 1) ? (h ? pc.w : pc.z) : (h ? pc.y : pc.x);
-                    constexpr int kHi = (int)0xF0F0F0F0u;
-                    bv = (long)(((unsigned long)(unsigned)(wd & kHi) << 32) |
-                                (unsigned)((wd << 4) & kHi));
-                } else {
-                    bv = h ? hi8(wr[U][c]) : lo8(wr[U][c]);
-                }
 #pragma unroll
-                for (int a = 0; a < AG; ++a) {
-                    d[h][a] = __builtin_amdgcn_mfma_i32_16x16x32_i8(
-                        h ? hi8(xr[U][c][a]) : lo8(xr[U][c][a]), bv, cinit, 0, 0, 0);
+                for (int t = 0; t < NT; ++t) {
+                    long bv;
                     if constexpr (W4) {
+                        const v4i pc = wr[U][t][c >> 1];
+                        const int wd = (c & 1) ? (h ? pc.w : pc.z) : (h ? pc.y : pc.x);
+                        constexpr int kHi = (int)0xF0F0F0F0u;
+                        bv = (long)(((unsigned long)(unsigned)(wd & kHi) << 32) |
+                                    (unsigned)((wd << 4) & kHi));
+                    } else {
+                        bv = h ? hi8(wr[U][t][c]) : lo8(wr[U][t][c]);
+                    }
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) d[h][a][i] >>= 4;
+                    for (int a = 0; a < AG; ++a) {
+                        d[h][a][t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(
+                            h ? hi8(xr[U][c][a]) : lo8(xr[U][c][a]), bv, cinit, 0, 0, 0);
+                        if constexpr (W4) {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) d[h][a][t][i] >>= 4;
+                        }
                     }
                 }
             }
@@ -277,8 +289,10 @@ __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
                 const size_t p = (size_t)(4 * (L + RL) + c);
                 if (!W4 || (c & 1)) {
                     const int pi = W4 ? c >> 1 : c;
-                    wr[U][pi] = __builtin_nontemporal_load(
-                        at(wp + ((size_t)(L + RL) * LB + pi * 64) * 16, wl));
+#pragma unroll
+                    for (int t = 0; t < NT; ++t)
+                        wr[U][t][pi] = __builtin_nontemporal_load(
+                            at(wp[t] + ((size_t)(L + RL) * LB + pi * 64) * 16, wl));
                 }
 #pragma unroll
                 for (int a = 0; a < AG; ++a) xr[U][c][a] = *at(ap + p * cs, al[a]);
@@ -287,32 +301,39 @@ __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
             for (int h = 0; h < 2; ++h) {
                 const int b = 8 * L + 2 * c + h;
                 if (!decltype(check)::value || b < nb) {
-                    const unsigned word = (unsigned)sr[U][c];
-                    const float ds = f16_bits_to_f32(h ? (word >> 16) : (word & 0xFFFFu));
 #pragma unroll
-                    for (int a = 0; a < AG; ++a) {
+                    for (int t = 0; t < NT; ++t) {
+                        const unsigned word = (unsigned)sr[U][t][c];
+                        const float ds = f16_bits_to_f32(h ? (word >> 16) : (word & 0xFFFFu));
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int dv = d[h][a][i];
-                            float tm = (W4 ? (float)dv : __int_as_float(dv) - kDotBiasF) *
-                                       sa[a][i];
-                            tm = tm * ds;
-                            fs[a][i] = fs[a][i] + tm;
-                        }
-                        if constexpr (DEBUG) {
+                        for (int a = 0; a < AG; ++a) {
 #pragma unroll
                             for (int i = 0; i < 4; ++i) {
-                                const int m = 16 * (a0 + a) + 4 * g + i;
-                                if (m < M && n < N)
-                                    block_dots[((size_t)m * N + n) * nb + b] =
-                                        W4 ? d[h][a][i] : d[h][a][i] - kDotBias;
+                                const int dv = d[h][a][t][i];
+                                float tm = (W4 ? (float)dv : __int_as_float(dv) - kDotBiasF) *
+                                           sa[a][i];
+                                tm = tm * ds;
+                                fs[a][t][i] = fs[a][t][i] + tm;
+                            }
+                            if constexpr (DEBUG) {
+#pragma unroll
+                                for (int i = 0; i < 4; ++i) {
+                                    const int m = 16 * (a0 + a) + 4 * g + i;
+                                    if (m < M && n[t] < N)
+                                        block_dots[((size_t)m * N + n[t]) * nb + b] =
+                                            W4 ? d[h][a][t][i] : d[h][a][t][i] - kDotBias;
+                                }
                             }
                         }
                     }
                 }
             }
         }
-        if (refill) sr[U] = *at(wp + (size_t)(L + RL) * LB * 16, sl);
+        if (refill) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+                sr[U][t] = *at(wp[t] + (size_t)(L + RL) * LB * 16, sl);
+        }
         // keep the next lap's uses of its (younger) loads below this point
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -329,14 +350,17 @@ __global__ __launch_bounds__(TPW * kWave) void k_skinny_q8_0(
             if (u < rem) lap(k * RL + u, u, false, T1{});
         });
     }
-    if (n >= N) return;
 #pragma unroll
-    for (int a = 0; a < AG; ++a)
+    for (int t = 0; t < NT; ++t) {
+        if (n[t] >= N) continue;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int m = 16 * (a0 + a) + 4 * g + i;
-            if (m < M) out[(size_t)m * N + n] = fs[a][i];
-        }
+        for (int a = 0; a < AG; ++a)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int m = 16 * (a0 + a) + 4 * g + i;
+                if (m < M) out[(size_t)m * N + n[t]] = fs[a][t][i];
+            }
+    }
 }
 
 template <int MT, int NT, int U, int S>
@@ -370,30 +394,22 @@ mri_status launch_i8_rows(const int8_t *act, size_t m, size_t kp, const float *s
     return launch_i8<MT, 1, 4, 4>(act, m, kp, sa_ptr, sa_stride, sa_value, w, out, acc_out, s);
 }
 
+template <int I>
+using Int = std::integral_constant<int, I>;
+
 // AG activation groups per wave, ns waves per tile (AG * ns groups of 16 rows).
-template <int AG, int TPW, int RL, int CS, bool DEBUG, bool W4>
-void launch_q8_w(const int8_t *act, size_t m, size_t kp, const float *sa_rows,
-                 const Q8MatrixDev &w, float *out, int32_t *block_dots, int ns, int mg,
-                 hipStream_t s) {
+template <int AG, int NT, int RL, int CS, bool DEBUG, bool W4>
+void launch_q8(const int8_t *act, size_t m, size_t kp, const float *sa_rows,
+               const Q8MatrixDev &w, float *out, int32_t *block_dots, int ns, int mg,
+               hipStream_t s) {
     const int G = (int)w.laps_per_tile();
-    const size_t waves = w.n_tiles * (size_t)ns;
-    size_t grid = (waves + TPW - 1) / TPW;
-    if (ns > TPW) grid = (grid + 7) / 8 * 8;  // XCD-major mapping (whole waves past the end exit)
-    hipLaunchKernelGGL((k_skinny_q8_0<AG, TPW, RL, CS, DEBUG, W4>),
-                       dim3((unsigned)grid), dim3(TPW * kWave), 0, s,
+    size_t grid = (w.n_tiles + NT - 1) / NT * (size_t)ns;
+    if (ns > 1) grid = (grid + 7) / 8 * 8;  // XCD-major mapping (whole waves past the end exit)
+    hipLaunchKernelGGL((k_skinny_q8_0<AG, NT, RL, CS, DEBUG, W4>),
+                       dim3((unsigned)grid), dim3(kWave), 0, s,
                        act, (int)m, (int)kp, sa_rows, reinterpret_cast<const v4i *>(w.laps),
                        (int)w.n_out, (int)w.n_tiles, G,
                        (int)w.n_blocks, out, block_dots, ns, mg);
-}
-
-template <int AG, int TPW, int RL, int CS, bool DEBUG>
-void launch_q8(const int8_t *act, size_t m, size_t kp, const float *sa_rows,
-               const Q8MatrixDev &w, float *out, int32_t *block_dots, int ns, int mg,
-                 hipStream_t s) {
-    if (w.w4)
-        launch_q8_w<AG, TPW, RL, CS, DEBUG, true>(act, m, kp, sa_rows, w, out, block_dots, ns, mg, s);
-    else
-        launch_q8_w<AG, TPW, RL, CS, DEBUG, false>(act, m, kp, sa_rows, w, out, block_dots, ns, mg, s);
 }
 
 }  // namespace
@@ -421,36 +437,64 @@ mri_status launch_skinny_int8(const int8_t *act, size_t m, const float *sa_ptr,
 
 namespace {
 
-// A wave takes AG groups of 16 rows of one tile; the ns waves of a tile share
-// a workgroup (four of them, above 32 rows) and so its weights in the CU's L1.
-// Groups a wave: two where that still leaves a wave for every SIMD (the
-// weight operand then feeds two MFMAs), else one, and one for W4, whose
-// weights cost half the bytes (us a call, two / one: Q8_0 100 x 4096 x 4096
-// 21.0 / 22.7, 100 x 4096 x 11008 43.3 / 46.8, 64 x 4096 x 4096 18.9 / 16.0,
-// 100 x 1024 x 1024 9.7 / 8.2, 32 x 4096 x 11008 20.9 / 23.5, 24 x 4096 x 4096
-// 17.6 / 13.6; W4 100 x 11008 x 4096 51.4 / 42.9, 32 x 4096 x 11008 22.0 /
-// 19.5).  With the activations in row groups (1 KiB a load) two tiles a wave,
-// which halved the row-strided loads, are no longer faster: 100 x 4096 x 4096
-// 30.9 in rows and two tiles, 21.0 now; 16 x 4096 x 11008 16.9, 15.4 now.
-template <int RL2, int RL1, bool DEBUG>
+// A wave takes AG groups of 16 rows of NT tiles; the waves of a tile are
+// neighbouring workgroups of one XCD and share its weights in L2 (four of them
+// in one workgroup: 2-10 % slower).  More groups a wave feed one weight
+// operand to more MFMAs, more tiles one activation operand; fewer leave more
+// waves, which 16 x 16 outputs a SIMD (u) decides.  us a call at K = 4096,
+// AG x NT = 1 x 1 / 2 x 1 / 2 x 2 / 4 x 2, the best marked:
+//   Q8_0    64 rows, 256 tiles (u = 1)    15.2* 19    -     -
+//          128 rows, 256 tiles (u = 2)    22.4  19.5*  -     -
+//           64 rows, 688 tiles (u = 2.7)   -    28.0* 28.8   -
+//          100 rows, 688 tiles (u = 4.7)   -    41.4  38.8*  -
+//           64 rows, 2000 tiles (u = 8)    -     -    49.8*  -
+//          128 rows, 2000 tiles (u = 16)   -     -    84.7  74.1*
+//         2048 rows, 688 tiles (u = 86)    -     -    418   357*
+//   W4, whose weights cost half the bytes,
+//           64 rows, 688 tiles (u = 2.7)  26.3* 26.9   -     -
+//          127 rows, 688 tiles (u = 5.4)   -    38.1* 40.9   -
+//          127 rows, 2000 tiles (u = 16)   -     -    85.3  79.1*
+// Up to 16 rows, two tiles of Q8_0 from one wave a SIMD on (5 x 4096 x 22016
+// 24.7 and 22.4).  Laps in flight of one group and tile: three, or two where K
+// is eight laps or less (64 x 2048 x 4096 12.0 and 11.3) and W4 has several
+// waves a SIMD (10 x 4096 x 20000 22.3 and 20.0).
+// Before, with one tile a wave and one or two groups at every size, 2048 x 4096 x
+// 11008 took 618 us and 127 x 4096 x 32000 111; now 368 and 77.
+template <bool DEBUG>
 void launch_q8_groups(const int8_t *act, size_t m, size_t kp, const float *sa_rows,
                       const Q8MatrixDev &w, float *out, int32_t *block_dots, int mg,
                       hipStream_t s) {
-    const int n1 = (int)((m + 15) / 16), n2 = (int)((m + 31) / 32);
-    const size_t simds = 4 * (size_t)std::max(device_cus(), 1);
-    const bool one = w.w4 || w.n_tiles * (size_t)n1 <= simds;
-    if (m <= 16 && mg == 1)
-        launch_q8<1, 1, RL1, 1024, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, 1, mg, s);
-    else if (m <= 16)
-        launch_q8<1, 1, RL1, 64, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, 1, mg, s);
-    else if (m <= 32 && one)
-        launch_q8<1, 2, RL1, 0, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, 2, mg, s);
-    else if (m <= 32)
-        launch_q8<2, 1, RL2, 0, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, 1, mg, s);
-    else if (one)
-        launch_q8<1, 4, RL2, 0, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, n1, mg, s);
-    else
-        launch_q8<2, 4, RL2, 0, DEBUG>(act, m, kp, sa_rows, w, out, block_dots, n2, mg, s);
+    auto go = [&](auto ag, auto nt, auto rl, auto cs) {
+        constexpr int AG = decltype(ag)::value;
+        const int ns = (int)((m + 16 * AG - 1) / (16 * AG));
+        auto run = [&](auto w4) {
+            launch_q8<AG, decltype(nt)::value, decltype(rl)::value, decltype(cs)::value, DEBUG,
+                      decltype(w4)::value>(act, m, kp, sa_rows, w, out, block_dots, ns, mg, s);
+        };
+        constexpr bool q8_only = AG < decltype(nt)::value;
+        if constexpr (!q8_only)
+            if (w.w4) return run(std::true_type{});
+        run(std::false_type{});
+    };
+    const Int<0> any{};
+    const Int<1> one{};
+    const Int<2> two{};
+    const double u = (double)w.n_tiles * ((m + 15) / 16) / (4 * std::max(device_cus(), 1));
+    if (m <= 16 && mg != 1) return go(one, one, two, Int<64>{});
+    if constexpr (!DEBUG) {
+        const bool laps2 = w.laps_per_tile() <= 8;
+        if (m <= 16) {
+            const Int<1024> group{};
+            if (u > 1 && !w.w4) return go(one, two, two, group);
+            return laps2 || u > 1 ? go(one, one, two, group) : go(one, one, Int<3>{}, group);
+        }
+        if (u <= (w.w4 ? 3 : 1))
+            return laps2 ? go(one, one, two, any) : go(one, one, Int<3>{}, any);
+        if (u > 12) return go(Int<4>{}, two, one, any);
+        if (u > (w.w4 ? 6.5 : 3.5)) return go(two, two, two, any);
+    }
+    // (the block dots' registers leave room for no more)
+    return u <= 1 ? go(one, one, two, any) : go(two, one, two, any);
 }
 
 }  // namespace
@@ -461,9 +505,9 @@ mri_status launch_skinny_q8_0(const int8_t *act, size_t m,
                               hipStream_t s, size_t mg) {
     if (w.n_tiles == 0 || m == 0) return MRI_OK;
     if (block_dots)
-        launch_q8_groups<2, 2, true>(act, m, w.kp, sa_rows, w, out, block_dots, (int)mg, s);
+        launch_q8_groups<true>(act, m, w.kp, sa_rows, w, out, block_dots, (int)mg, s);
     else
-        launch_q8_groups<2, 3, false>(act, m, w.kp, sa_rows, w, out, nullptr, (int)mg, s);
+        launch_q8_groups<false>(act, m, w.kp, sa_rows, w, out, nullptr, (int)mg, s);
     MRI_LAUNCHED("k_skinny_q8_0");
     return MRI_OK;
 }
