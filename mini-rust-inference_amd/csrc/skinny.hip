@@ -376,22 +376,32 @@ mri_status launch_i8(const int8_t *act, size_t m, size_t kp, const float *sa_ptr
     MRI_LAUNCHED("k_skinny_int8");
     return MRI_OK;
 }
-// Tiles and waves of a workgroup.  From 512 tiles, four tiles share each
-// activation load: the tiles' reads of the rows from L2 are what bounds the
-// kernel there (60 x 4096 x 11008: 35.3 us one tile each, 25.5 four).  Below,
-// one tile and as many waves as K has work for (24 x 4096 x 4096 with its
-// quantization: 15.4 us one wave, 13.3 four, 12.5 sixteen; 12 x 512 x 2048: 6.4
-// four, 7.6 sixteen).
+// Tiles and waves of a workgroup.  One tile while every CU has at most one
+// workgroup, two up to two tiles a CU, then four: tiles that share a workgroup
+// share its activation loads from L2, which bound the kernel, but 5 rows to 63
+// fill a CU with one workgroup (us a call from f32, NT = 1 / 2 / 4: 32 x 5120 x
+// 5120 25.4 / 17.8 / 21.1, 63 x 4096 x 8192 - / 21.0 / 24.3, 63 x 4096 x 11008
+// - / 31.6 / 25.1; four from 512 tiles on, as before, 25.5 at 63 x 4096 x 8192).
+// Waves: eight of two chunks in flight (32 x 11008 x 4096 23.8, sixteen 25.0;
+// four tiles: four waves); for one tile of rows sixteen where K is 48 to 128
+// chunks (5 x 4096 x 4096 9.4, eight 9.9) and four of four below (16 x 512 x
+// 2048 7.0, 7.1).
 template <int MT>
 mri_status launch_i8_rows(const int8_t *act, size_t m, size_t kp, const float *sa_ptr,
                           int sa_stride, float sa_value, const QMatrixDev &w, float *out,
                           int32_t *acc_out, hipStream_t s) {
-    const size_t chunks = w.kp / kChunkK;
-    if (w.n_tiles >= 512)
-        return launch_i8<MT, 4, 4, 4>(act, m, kp, sa_ptr, sa_stride, sa_value, w, out, acc_out, s);
-    if (chunks >= 48)
-        return launch_i8<MT, 1, 2, 16>(act, m, kp, sa_ptr, sa_stride, sa_value, w, out, acc_out, s);
-    return launch_i8<MT, 1, 4, 4>(act, m, kp, sa_ptr, sa_stride, sa_value, w, out, acc_out, s);
+    const size_t chunks = w.kp / kChunkK, cus = (size_t)std::max(device_cus(), 1);
+    if (w.n_tiles > 2 * cus)
+        return launch_i8<MT, 4, 2, 4>(act, m, kp, sa_ptr, sa_stride, sa_value, w, out, acc_out, s);
+    if (w.n_tiles > cus)
+        return launch_i8<MT, 2, 2, 8>(act, m, kp, sa_ptr, sa_stride, sa_value, w, out, acc_out, s);
+    if constexpr (MT == 1) {
+        if (chunks < 48)
+            return launch_i8<1, 1, 4, 4>(act, m, kp, sa_ptr, sa_stride, sa_value, w, out, acc_out, s);
+        if (chunks < 128)
+            return launch_i8<1, 1, 2, 16>(act, m, kp, sa_ptr, sa_stride, sa_value, w, out, acc_out, s);
+    }
+    return launch_i8<MT, 1, 2, 8>(act, m, kp, sa_ptr, sa_stride, sa_value, w, out, acc_out, s);
 }
 
 template <int I>

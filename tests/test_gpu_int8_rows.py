@@ -20,6 +20,8 @@ pytestmark = pytest.mark.gpu
     (20, 70, 3072), (49, 50, 4111),                      # 16 waves
     (6, 8192, 64), (31, 8177, 200), (40, 8200, 72), (63, 8193, 1028),  # four tiles
     (16, 24, 4096), (17, 24, 4096),                      # one pass, two launches
+    (5, 4200, 1000), (30, 8000, 320), (63, 4113, 3000),  # two tiles a workgroup
+    (7, 40, 8256), (40, 20, 8300),                       # one tile, long K
 ])
 def test_rows_bit_exact(m, n, k):
     import mri_qmatmul as M
