@@ -496,7 +496,8 @@ void launch_q8_groups(const int8_t *act, size_t m, size_t kp, const float *sa_ro
         if (m <= 16) {
             const Int<1024> group{};
             if (u > 1 && !w.w4) return go(one, two, two, group);
-            return laps2 || u > 1 ? go(one, one, two, group) : go(one, one, Int<3>{}, group);
+            if (u <= 1 && !laps2) return go(one, one, Int<3>{}, group);
+            if (u <= 1024) return go(one, one, two, group);  // (2^30 channels: past the grid)
         }
         if (u <= (w.w4 ? 3 : 1))
             return laps2 ? go(one, one, two, any) : go(one, one, Int<3>{}, any);

@@ -46,6 +46,9 @@ def check(got, x, raw, n, k):
 @pytest.mark.parametrize("m,n,k", [
     (1, 33, 96), (2, 16, 32), (2, 40, 1056), (3, 50, 544), (4, 25, 4128),  # per block
     (1, 70, 8224), (3, 31, 8192), (1, 20, 32768),      # 16 waves; past its LDS
+    (2, 33, 14336), (4, 20, 11008), (3, 17, 30016), (2, 40, 27488),  # LDS in parts
+    (1, 2500, 8192), (1, 2500, 8448), (1, 3300, 12288),  # staged or per block
+    (2, 4100, 2048), (2, 4150, 4096), (2, 40, 8192), (2, 1030, 14336),  # two rows staged
     (3, 6200, 64),                                     # tiled from 3 rows on
     (5, 1, 32), (16, 17, 288), (7, 6200, 544),          # 16-row tiles, narrow and wide
     (17, 33, 32), (32, 31, 288), (18, 8300, 320),       # 32-row tiles

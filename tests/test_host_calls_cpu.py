@@ -122,6 +122,19 @@ def check_q4_0_grids(h):
             assert need <= got < need + 8, (m, k, n, launched)
 
 
+def check_q4_0_long_rows(h):
+    """Two to four rows whose planes exceed LDS, and a row of few channels, do
+    not take the form that was slower for them (kernels of 16 x 16 tiles, and a
+    workgroup for 16 channels)."""
+    for m, k, n in ((2, 14336, 4096), (2, 28672, 8192), (4, 11008, 4096), (1, 28672, 8192)):
+        (name, _), = h.q4_0(m, k, n)
+        assert "k_q4_0_gemv" in name, (m, k, n)
+    for m, k, n in ((1, 8192, 1024), (1, 8192, 4352), (1, 14336, 2048), (1, 16384, 6144),
+                    (2, 8192, 4352), (2, 10240, 5120), (2, 14336, 2048)):
+        (name, _), = h.q4_0(m, k, n)
+        assert "k_q4_0_lds" in name, (m, k, n)
+
+
 def check_block_grids(h):
     """As above, for the quantized rows of W4A8 past the LDS-tiled kernel."""
     for m, n in ((2**21, 2**13), (2**21 + 5, 2**13 + 1), (2**17, 2**17), (16, 2**30), (32, 2**30)):
