@@ -39,8 +39,8 @@
  * Concurrency: calls are asynchronous on `stream`.  Handles are immutable
  * after creation and may be shared by calls on any stream.  Internal scratch
  * (activation quantization, the prefill GEMMs' partial tiles and tile
- * counters) is kept per (device, stream), so concurrent calls on different
- * streams do not interfere.
+ * counters, Q4_0's K parts) is kept per (device, stream), so concurrent calls
+ * on different streams do not interfere.
  */
 #ifndef MRI_QMATMUL_H
 #define MRI_QMATMUL_H
@@ -216,7 +216,9 @@ mri_status mri_matmul_q8_0_direct_noalloc(const float *input, const size_t *dims
  * 2i = low nibble of byte i minus 8, element 2i+1 = high nibble minus 8).
  * Check order as the reference: ndim != 2 -> InvalidShape; dims[1] != k ->
  * ShapeMismatch; k % 32 -> InvalidShape; len != n_out*(k/32)*18 ->
- * InvalidShape.  out is [m, n_out] f32. */
+ * InvalidShape.  out is [m, n_out] f32.
+ * From 33 rows a call may take a workspace for K parts (at most 128 MiB a
+ * stream, kept); without it, and under capture, it gives the same bits. */
 mri_status mri_matmul_q4_0_dequant(const float *input, const size_t *dims,
                                    size_t ndim, const uint8_t *weight_q4,
                                    size_t weight_len, size_t n_out, size_t k,

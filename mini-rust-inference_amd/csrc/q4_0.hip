@@ -19,8 +19,10 @@
 // the activations of block 4 lap + g and is zero elsewhere; the four MFMAs
 // add up to register p of lane (r, g) = plane p's sum of its own block, which
 // it adds (smallest first) and scales by the d that it loaded.  The planes
-// are split once per workgroup into LDS, in parts where K is too long for it; bits below 2^-133, which they do not
-// hold, are added in f32 where there are any (as in q4_gemm.hip).  Bound: the unpacking (2.6 VALU
+// are split once per workgroup into LDS, in parts where K is too long for it;
+// bits below 2^-133, which they do not hold, are added in f32 where there are
+// any (as in q4_gemm.hip; 0.1-0.25 us a call for seeing that there are none).
+// Bound: the unpacking (2.6 VALU
 // operations a weight) and its loads, 72-byte pieces of 16 rows.  It took
 // 1 x 4128 x 11008 from 23.4 to 10.4 us (the earlier two-lanes-a-block f32
 // kernel), 2 x 4128 x 8000 from 33.1 to 9.2 and 4 x 992 x 512 from 12.9 to

@@ -22,7 +22,8 @@
 // makes the 16-row fragment reads conflict-free.
 //
 // Bound: the three MFMAs (1536 cycles a SIMD and block of a 128 x 256 tile)
-// and the splitting, unpacking and folding (about as many VALU cycles), which
+// and the splitting, unpacking and folding (as many VALU cycles: 43 and 44 % of
+// the kernel's, by the counters, where there is a workgroup), which
 // the barrier keeps apart: 256 x 4096 x 11008 takes 88 us (263 TFLOP/s of
 // f32 products, 0.79 PFLOP/s of bf16 ones); the kernel before it, one wave a
 // weight row on the f32 VALU, took 3693 us.  Loading two stages ahead instead
@@ -436,7 +437,7 @@ constexpr int kMaxParts = 8, kMinPartBlocks = 8;
 // part order), so they depend on the sizes alone; *whole is the better of the
 // first two tiles for one workgroup that takes all parts (the third one's
 // registers do not hold their totals too: 333 x 4096 x 12288 430 us, in
-// 128 x 128 tiles 215; split 143).
+// 128 x 128 tiles 215; split 133).
 void plan_q4(size_t m, size_t k, size_t n, int *tile, int *parts, int *whole) {
     const long long nb = (long long)(k / 32), cus = std::max(device_cus(), 1);
     long long best = -1, best_whole = -1;
@@ -482,7 +483,7 @@ mri_status launch_gemm(const float *x, size_t m, size_t k, const uint8_t *w, siz
         // A stream that is being captured gets no K split over workgroups: no
         // recorded graph holds the workspace, which may therefore grow at any
         // later call.  One workgroup a tile adds the same parts instead (split
-        // and not: 256 x 4096 x 11008 98 and 116 us, 64 x 4096 x 4096 20 and 74).
+        // and not: 256 x 4096 x 11008 88 and 107 us, 64 x 4096 x 4096 19 and 77).
         void *ws = nullptr;
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
